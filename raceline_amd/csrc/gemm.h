@@ -37,6 +37,12 @@ int run_gemm4(int book, const _Float16 *x, int x_stride, int M, int K, int N, co
               const float *srow, float *y, int y_stride, int accum, int *cnt, void *ws, size_t ws_bytes,
               hipStream_t st);
 
+// The kernel for calls with too few 128 x 256 tiles (gemm_mid.hip): gemm_mid_tiles gives the
+// 32-row tiles (1 or 2) of its workgroups' rows, or 0 where gemm4_kernel takes the call. Both
+// kernels give the same bits.
+int gemm_mid_tiles(int M, int K, int N, int S);
+int launch_gemm_mid(int book, int sd, int mt, const GemmArgs &a, int S, int accum, hipStream_t st);
+
 // defined in linear.hip
 void launch_group_sums(const _Float16 *x, int x_stride, int M, int K, float *gsT, int m_pad, hipStream_t st);
 void launch_row_sums(const float *gsT, int G, int m_pad, int M, float *asum, hipStream_t st);

@@ -1,4 +1,5 @@
-// Prefill GEMM on gfx950 for the 4-bit formats (affine and native codebooks), M > 8.
+// Prefill GEMM on gfx950 for the 4-bit formats (affine and native codebooks), M > 8, where its
+// workgroup tiles fill the chip (gemm_mid.hip takes smaller calls, with the same bits).
 //
 //   affine: y[m][n] = sum_g s[n][g] * (x_g . q_g)[m][n] + b[n][g] * gsum[m][g]
 //   native: y[m][n] = s[n] * (x . L(q))[m][n]  (+ 0.5 s[n] rowsum[m] for the half-step book)
@@ -246,10 +247,6 @@ struct StageSrc {
   bool a_row[4];
   int K, GP, G4, wave, lane;
 };
-
-__device__ __forceinline__ __attribute__((address_space(3))) void *lds_at(unsigned char *lds, int off) {
-  return (__attribute__((address_space(3))) void *)(lds + off);
-}
 
 // Loads group pair p into LDS stage `stage`: 4 activation chunks (16 bytes each), 2 code
 // chunks of 16 bytes (tile 2 wave + i: its pair-p kilobyte) and 2 scale words (quad p/2 of
@@ -790,6 +787,10 @@ int run_gemm4(int book, const _Float16 *x, int x_stride, int M, int K, int N, co
     if (a.gs) c.gs = a.gs + (size_t)r0 * a.gs_stride;
     if (a.rscale) c.rscale = a.rscale + r0;
     if (a.asum) c.asum = a.asum + r0;
+    if (const int mt = gemm_mid_tiles(c.M, K, N, S)) {   // too few of this kernel's tiles to fill the chip
+      if (int rc = launch_gemm_mid(book, sd, mt, c, S, accum, st)) return rc;
+      continue;
+    }
     const dim3 grid((c.M + kGM - 1) / kGM * nblocks, S);
     int rc;
     switch (book) {

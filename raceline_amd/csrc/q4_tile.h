@@ -119,6 +119,18 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, ui
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, (int)bytes, kBufFlags);
 }
 
+// The LDS address a LDS-DMA writes to.
+__device__ __forceinline__ __attribute__((address_space(3))) void *lds_at(unsigned char *lds, int off) {
+  return (__attribute__((address_space(3))) void *)(lds + off);
+}
+
+// One 16-byte-per-lane LDS-DMA into the kilobyte at lds + at. (Not a template: in one, an
+// argument of a dependent type makes the host pass refuse the 16-byte size and drop the
+// kernel's launch stub without a diagnostic.)
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, unsigned char *lds, int at, uint32_t voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds_at(lds, at), 16, voff, soff, 0, 0);
+}
+
 // acc + float(s16) * p with the 16-bit float taken from the low or high half of a packed pair
 template <int SD, int HI>
 __device__ __forceinline__ float fma_scale(uint32_t pr, float p, float acc) {
