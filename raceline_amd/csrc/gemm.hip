@@ -586,27 +586,34 @@ __global__ __launch_bounds__(kGThreads) void gemm4_kernel(GemmArgs a) {
   }
 
   // D of a 32x32 tile: lane l holds column l%32, rows 8 (v/4) + 4 (l/32) + v%4. acc becomes
-  // this split's values (split 0's with y added when asked).
-  const int n = n0 + 32 * wave + c32;
+  // this split's values (split 0's with y added when asked). Loads are clamped into the
+  // matrix and issued a token tile at a time, ahead of their use, and only the stores look at
+  // the edges: loading y inside a per-element branch waited for memory once per element,
+  // about 20 us per round of workgroups of a residual projection.
+  const int n = n0 + 32 * wave + c32, nc = min(n, a.N - 1);
   const bool col = n < a.N;
-  const float rs_n = BOOK == kAffine || !a.srow || !col ? 1.0f : a.srow[n];   // no row scales: the raw product
+  const float rs_n = BOOK == kAffine || !a.srow ? 1.0f : a.srow[nc];   // no row scales: the raw product
 #pragma unroll
   for (int mt = 0; mt < 4; ++mt) {
+    float yv[16];
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      const int m = m0 + mt * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-      if (col && m < a.M) {
-        float val = acc[mt][v];
-        if constexpr (BOOK == kAffine)   // undoes the prep's 2^e, exactly (the scale staged in the prologue)
-          val *= reinterpret_cast<const float *>(lds + kRscaleLds)[m - m0];
-        if constexpr (BOOK == kInt16) {
-          if (split == 0) val = __builtin_fmaf(0.5f, a.asum[m], val);
-        }
-        if constexpr (BOOK != kAffine) val *= rs_n;
-        if (acc_here) val = a.y[(size_t)m * a.y_stride + n] + val;
-        acc[mt][v] = val;
-      }
+      const int m = min(m0 + mt * 32 + 8 * (v >> 2) + 4 * h + (v & 3), a.M - 1);
+      if (acc_here) yv[v] = a.y[(size_t)m * a.y_stride + nc];
     }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      float val = acc[mt][v];
+      if constexpr (BOOK == kAffine)   // undoes the prep's 2^e, exactly (the scale staged in the prologue)
+        val *= reinterpret_cast<const float *>(lds + kRscaleLds)[mt * 32 + 8 * (v >> 2) + 4 * h + (v & 3)];
+      if constexpr (BOOK == kInt16) {
+        if (split == 0) val = __builtin_fmaf(0.5f, a.asum[min(m0 + mt * 32 + 8 * (v >> 2) + 4 * h + (v & 3), a.M - 1)], val);
+      }
+      if constexpr (BOOK != kAffine) val *= rs_n;
+      if (acc_here) val = yv[v] + val;
+      acc[mt][v] = val;
+    }
+    __builtin_amdgcn_sched_barrier(0);   // one token tile's loads at a time: all four's do not fit the registers
   }
   if (S == 1) {
     if (!col) return;
