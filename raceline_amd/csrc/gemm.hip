@@ -312,9 +312,10 @@ __device__ __forceinline__ int bias_piece_at(int pos, bool pro) {
 // A fragment of step j of a pair (see gemm4_kernel): token tile 2 ((j >> 3) & 1) + (j & 1),
 // 32 rows of 256 bytes apart per tile, chunk of step (j >> 1) & 3 of group j >> 4.
 template <int STAGE>
-__device__ __forceinline__ half8 read_frag(const unsigned char *lds, const uint32_t (&aoff)[2][4], int j) {
+__device__ __forceinline__ half8 read_frag(const unsigned char *lds, const uint32_t (&aoff)[2][2][4], int j) {
   const int gg = j >> 4, mt = 2 * ((j >> 3) & 1) + (j & 1), i = (j >> 1) & 3;
-  return *reinterpret_cast<const half8 *>(lds + a_part(STAGE) + mt * 32 * kARowBytes + aoff[gg][i]);
+  return *reinterpret_cast<const half8 *>(lds + (STAGE == 2 ? 0 : a_part(STAGE)) + mt * 32 * kARowBytes +
+                                          aoff[STAGE == 2][gg][i]);
 }
 
 template <int BOOK, int SD, bool ACC>
@@ -385,11 +386,18 @@ __global__ __launch_bounds__(kGThreads) void gemm4_kernel(GemmArgs a) {
   const int h = lane >> 5, c32 = lane & 31;
   const int tt = c32 >> 4, cr = c32 & 15;                 // 16-row tile within the 32, row in it
   const int kt = 2 * wave + tt;                           // the lane's 16-row tile in the workgroup
-  uint32_t aoff[2][4];                                    // A fragment offsets within a stage
+  // A fragment offsets within a stage, and the same from stage 2's part, 64 KB up: past the
+  // 16-bit immediate of an LDS read, so the reads of that stage took an address add each (34
+  // per pair, of its 239 VALU instructions) until it got base addresses of its own
+  uint32_t aoff[2][2][4];
 #pragma unroll
   for (int gg = 0; gg < 2; ++gg)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) aoff[gg][i] = (uint32_t)(c32 * kARowBytes + (((8 * gg + 2 * i + h) ^ cr) << 4));
+    for (int i = 0; i < 4; ++i) {
+      aoff[0][gg][i] = (uint32_t)(c32 * kARowBytes + (((8 * gg + 2 * i + h) ^ cr) << 4));
+      aoff[1][gg][i] = a_part(2) + aoff[0][gg][i];
+      asm volatile("" : "+v"(aoff[1][gg][i]));   // a register of its own
+    }
   const uint32_t boff = (uint32_t)(kt * 1024 + 256 * h + 16 * cr);   // within a stage's code part
   const uint32_t soff = (uint32_t)(kt * 256 + 16 * cr);               // within its scale part
 
