@@ -127,12 +127,21 @@ class RlqError(RuntimeError):
     pass
 
 
+_STATUS_FREE = ("rlq_abi_version", "rlq_set_fatal")   # int results that are no status
+
+
+@functools.lru_cache(maxsize=None)
+def _entry(name: str):
+    """(set_fatal, function, whether its int result is a status) of one entry point."""
+    lib = load()
+    return lib.rlq_set_fatal, getattr(lib, name), SIGNATURES[name][0] is c_int and name not in _STATUS_FREE
+
+
 def call(name: str, *args):
     """Calls rlq_<name> in non-fatal mode and raises RlqError on a nonzero status."""
-    lib = load()
-    lib.rlq_set_fatal(0)
-    rc = getattr(lib, name)(*args)
-    if isinstance(rc, int) and rc != 0 and SIGNATURES[name][0] is c_int and name not in (
-            "rlq_abi_version", "rlq_set_fatal"):
-        raise RlqError(f"{name}: {lib.rlq_last_error().decode(errors='replace')}")
+    set_fatal, fn, status = _entry(name)
+    set_fatal(0)
+    rc = fn(*args)
+    if status and rc != 0:
+        raise RlqError(f"{name}: {load().rlq_last_error().decode(errors='replace')}")
     return rc

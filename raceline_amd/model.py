@@ -11,6 +11,7 @@ import functools
 import torch
 
 from . import lib
+from .ops import _stream
 
 KINDS = {1: "q4a", 2: "q4n", 3: "q4a_rows", 4: "q4n_rows", 5: "f16b", 6: "f32"}
 
@@ -90,10 +91,6 @@ def copy_from_device_ptr(ptr: int, shape, dtype=torch.float32, device="cuda") ->
     if rc != 0:
         raise RuntimeError(f"hipMemcpy failed ({rc})")
     return out
-
-
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
 
 
 class Engine:

@@ -30,9 +30,18 @@ def _ptr(t) -> int:
     return 0 if t is None else t.data_ptr()
 
 
+# The current stream's handle without a Stream object around it: torch.cuda.current_stream()
+# took 2.7 of the 10.4 us of a one-token linear's call, this pair 0.2.
+_current_device = getattr(torch._C, "_cuda_getDevice", None)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(stream=None) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    if stream is not None:
+        return stream.cuda_stream
+    if _raw_stream is None or _current_device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_current_device())
 
 
 def scale_code(dtype: torch.dtype) -> int:
