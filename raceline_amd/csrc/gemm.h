@@ -43,6 +43,11 @@ int run_gemm4(int book, const _Float16 *x, int x_stride, int M, int K, int N, co
 int gemm_mid_tiles(int M, int K, int N, int S);
 int launch_gemm_mid(int book, int sd, int mt, const GemmArgs &a, int S, int accum, hipStream_t st);
 
+// The affine kernel for a few rows (gemm_few.hip), the same bits again, and whether it takes a
+// call; a.x: the prepped activations by chunk, then row ([K / 8][M][8 halves]).
+bool gemm_few_fits(int M, int N, int S);
+int launch_gemm_few(int sd, const GemmArgs &a, int S, int accum, hipStream_t st);
+
 // defined in linear.hip
 void launch_group_sums(const _Float16 *x, int x_stride, int M, int K, float *gsT, int m_pad, hipStream_t st);
 void launch_row_sums(const float *gsT, int G, int m_pad, int M, float *asum, hipStream_t st);

@@ -1,5 +1,5 @@
 // Prefill GEMM on gfx950 for the 4-bit formats (affine and native codebooks), M > 8, where its
-// workgroup tiles fill the chip (gemm_mid.hip takes smaller calls, with the same bits).
+// workgroup tiles fill the chip (gemm_mid.hip and gemm_few.hip take smaller calls, with the same bits).
 //
 //   affine: y[m][n] = sum_g s[n][g] * (x_g . q_g)[m][n] + b[n][g] * gsum[m][g]
 //   native: y[m][n] = s[n] * (x . L(q))[m][n]  (+ 0.5 s[n] rowsum[m] for the half-step book)
@@ -156,7 +156,9 @@ __device__ __forceinline__ int row_exponent(float mx) {
 // order, and each group's sum is its 8 threads' fixed butterfly whatever THR is). Rows of more
 // than 8192 activations take 1024 threads: with 256 threads, 16 chunks each held 154 VGPRs
 // (3 waves per SIMD), and the 27B down projection's prep (K = 17408) ran at 4.1 TB/s.
-template <int SD, int CPT, int THR = kPrepThreads>
+// COLS: the prepped row goes out by chunk, then row (chunk c of row m at (c M + m) 8 halves, the
+// order gemm_few_kernel reads), not by row.
+template <int SD, int CPT, int THR = kPrepThreads, bool COLS = false>
 __global__ __launch_bounds__(THR) void gemm_prep1_kernel(const _Float16 *x, int x_stride, int M, int K,
                                                          _Float16 *xp, uint16_t *gs, int gs_stride, float *rscale) {
   __shared__ float wmax[THR / 64];
@@ -190,7 +192,7 @@ __global__ __launch_bounds__(THR) void gemm_prep1_kernel(const _Float16 *x, int 
     sum += __shfl_xor(sum, 2);
     sum += __shfl_xor(sum, 4);
     if (c >= C) continue;
-    *reinterpret_cast<u32x4 *>(xp + (size_t)m * K + 8 * c) = prep_x8_scaled(v[j], f);
+    *reinterpret_cast<u32x4 *>(xp + (COLS ? ((size_t)c * M + m) * 8 : (size_t)m * K + 8 * c)) = prep_x8_scaled(v[j], f);
     if ((c & 7) == 0) write_gs_pieces<SD>(gs, gs_stride, m, c >> 3, G, sum);
   }
 }
@@ -201,7 +203,7 @@ __global__ __launch_bounds__(THR) void gemm_prep1_kernel(const _Float16 *x, int 
 // (coalesced 16-byte loads and stores); the 8 threads of a group add their partial sums
 // with a fixed butterfly. A row that is all zeros, or holds an infinity or a NaN, keeps
 // e = 0.
-template <int SD>
+template <int SD, bool COLS = false>
 __global__ __launch_bounds__(kPrepThreads) void gemm_prep_kernel(const _Float16 *x, int x_stride, int M, int K,
                                                                  _Float16 *xp, uint16_t *gs, int gs_stride,
                                                                  float *rscale) {
@@ -233,7 +235,7 @@ __global__ __launch_bounds__(kPrepThreads) void gemm_prep_kernel(const _Float16 
     sum += __shfl_xor(sum, 2);
     sum += __shfl_xor(sum, 4);
     if (!in) continue;
-    *reinterpret_cast<u32x4 *>(xp + (size_t)m * K + 8 * c) = prep_x8_scaled(v, f);
+    *reinterpret_cast<u32x4 *>(xp + (COLS ? ((size_t)c * M + m) * 8 : (size_t)m * K + 8 * c)) = prep_x8_scaled(v, f);
     if ((c & 7) == 0) write_gs_pieces<SD>(gs, gs_stride, m, c >> 3, G, sum);
   }
 }
@@ -756,6 +758,9 @@ int run_gemm4(int book, const _Float16 *x, int x_stride, int M, int K, int N, co
   a.srow = srow;
   a.y = y;
   a.M = M; a.K = K; a.N = N; a.y_stride = y_stride;
+  const int S = gemm_split_of(K, N);
+  RLQ_REQUIRE(S == 1 || cnt, "prefill kernel: this weight splits K in %d, which needs the workspace's counters", S);
+  const bool few = book == kAffine && gemm_few_fits(M, N, S);
   if (book == kAffine) {
     const int gs_stride = gs_stride_of(G, sd);
     _Float16 *xp = static_cast<_Float16 *>(ws);
@@ -767,7 +772,11 @@ int run_gemm4(int book, const _Float16 *x, int x_stride, int M, int K, int N, co
 #define RLQ_PREP(THR, KERNEL, ...)                                                                                     \
   (sd == RLQ_BF16 ? KERNEL<1, ##__VA_ARGS__><<<M, THR, 0, st>>>(x, x_stride, M, K, xp, gs, gs_stride, rscale)          \
                   : KERNEL<0, ##__VA_ARGS__><<<M, THR, 0, st>>>(x, x_stride, M, K, xp, gs, gs_stride, rscale))
-    if (cpt <= 4) RLQ_PREP(kPrepThreads, gemm_prep1_kernel, 4);
+    if (few) {   // by chunk, then row
+      if (cpt <= 4) RLQ_PREP(kPrepThreads, gemm_prep1_kernel, 4, kPrepThreads, true);
+      else if (cpt <= 16) RLQ_PREP(1024, gemm_prep1_kernel, 4, 1024, true);
+      else RLQ_PREP(kPrepThreads, gemm_prep_kernel, true);
+    } else if (cpt <= 4) RLQ_PREP(kPrepThreads, gemm_prep1_kernel, 4);
     else if (cpt <= 16) RLQ_PREP(1024, gemm_prep1_kernel, 4, 1024);   // K <= 32768: 4 chunks per thread of 1024
     else RLQ_PREP(kPrepThreads, gemm_prep_kernel);
 #undef RLQ_PREP
@@ -784,8 +793,6 @@ int run_gemm4(int book, const _Float16 *x, int x_stride, int M, int K, int N, co
       a.asum = asum;
     }
   }
-  const int S = gemm_split_of(K, N);
-  RLQ_REQUIRE(S == 1 || cnt, "prefill kernel: this weight splits K in %d, which needs the workspace's counters", S);
   a.np_split = ((G + 1) / 2 + S - 1) / S;
   a.cnt = cnt;
   if (S > 1) a.y_part = reinterpret_cast<float *>(static_cast<char *>(ws) + books_workspace(book, M, K));
@@ -802,6 +809,10 @@ int run_gemm4(int book, const _Float16 *x, int x_stride, int M, int K, int N, co
     if (a.gs) c.gs = a.gs + (size_t)r0 * a.gs_stride;
     if (a.rscale) c.rscale = a.rscale + r0;
     if (a.asum) c.asum = a.asum + r0;
+    if (few) {   // 256 tiles of 32 x 32 at most: never more than one chunk
+      if (int rc = launch_gemm_few(sd, c, S, accum, st)) return rc;
+      continue;
+    }
     if (const int mt = gemm_mid_tiles(c.M, K, N, S)) {   // too few of this kernel's tiles to fill the chip
       if (int rc = launch_gemm_mid(book, sd, mt, c, S, accum, st)) return rc;
       continue;

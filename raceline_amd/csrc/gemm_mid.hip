@@ -17,6 +17,7 @@
 //  - The MFMAs of a group run beside the scale FMAs of the group (or row tile) before it and
 //    the code conversion of the group after it.
 #include "gemm.h"
+#include "gemm_bias.h"
 #include "q4_tile.h"
 #include "../../include/rlq.h"
 
@@ -29,8 +30,8 @@ namespace rlq {
 constexpr int kMidWaves = 4;             // (two per workgroup measured the same on small grids, up to 1.6 times slower on full ones)
 constexpr int kMidCols = 32 * kMidWaves; // features of a workgroup
 constexpr int kMidRow = 256;             // LDS bytes of one row of a stage: one pair of groups, 128 fp16
-constexpr int kMidBiasPro = 11;          // bias steps before the K loop, as gemm4_kernel runs them
-constexpr int kMidBiasChunk = 8;         // bias steps loaded at a time after it
+constexpr int kBiasSrcPro = 11;          // bias steps before the K loop, as gemm4_kernel runs them
+constexpr int kBiasSrcChunk = 8;         // bias steps loaded at a time after it
 
 template <int MT> constexpr int mid_stage_bytes() { return 32 * MT * kMidRow; }
 
@@ -75,56 +76,6 @@ __device__ __forceinline__ void mid_rows(const MidSrc<DMA> &src, unsigned char *
   for (int i = 0; i < DMA; ++i)   // the rows of DMA i are 16 i past DMA 0's: the same logical chunk
     dma16(rx, lds, s * mid_stage_bytes<MT>() + (src.wave + kMidWaves * i) * 1024,
           tail && (src.c0 & 8) ? kFarOffset : src.aoff[i], 256 * p);
-}
-
-// C steps of the bias product (see the kernel): the pieces of the wave's rows and its
-// features' scale quads, all requested at once.
-struct MidBias {
-  __amdgpu_buffer_rsrc_t rgs, rsb;
-  uint32_t svoff;
-  int M, gs_stride, G4, m0, c32, h;
-};
-
-template <int SD, int MT, int C>
-__device__ __forceinline__ void mid_bias_load(const MidBias &b, u32x4 (&bv)[C], u32x4 (&ba)[C][MT], int st0, int st1) {
-#pragma unroll
-  for (int u = 0; u < C; ++u) {
-    const int st = st0 + u, q = SD == 0 ? 2 * st + b.h : st;            // quad of groups 4q .. 4q+3
-    bv[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                          b.rsb, st < st1 && q < b.G4 ? b.svoff + 256u * q : kFarOffset, 0, 0));
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int m = b.m0 + 32 * mt + b.c32;
-      const uint32_t off = (uint32_t)(((size_t)m * b.gs_stride + 16 * st + 8 * b.h) * 2);
-      ba[u][mt] = __builtin_bit_cast(
-          u32x4, __builtin_amdgcn_raw_buffer_load_b128(b.rgs, st < st1 && m < b.M ? off : kFarOffset, 0, 0));
-    }
-  }
-}
-
-template <int SD, int MT, int C>
-__device__ __forceinline__ void mid_bias_mul(const u32x4 (&bv)[C], const u32x4 (&ba)[C][MT], int h, f32x16 (&acc)[MT]) {
-#pragma unroll
-  for (int u = 0; u < C; ++u) {
-    u32x4 d;
-    if constexpr (SD == 0) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) d[e] = (bv[u][e] >> 16) * 0x10001u;       // (b, b): times hi and lo
-    } else {
-      const uint32_t b0 = (h ? bv[u][2] : bv[u][0]) >> 16, b1 = (h ? bv[u][3] : bv[u][1]) >> 16;
-      d[0] = d[1] = b0 * 0x10001u;                                          // b of group 4q + 2h, four times
-      d[2] = d[3] = b1 * 0x10001u;                                          // and of group 4q + 2h + 1
-    }
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      if constexpr (SD == 0)
-        acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, ba[u][mt]),
-                                                        __builtin_bit_cast(half8, d), acc[mt], 0, 0, 0);
-      else
-        acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ba[u][mt]),
-                                                         __builtin_bit_cast(bf16x8, d), acc[mt], 0, 0, 0);
-    }
-  }
 }
 
 template <int BOOK, int SD, int MT, int R>
@@ -200,15 +151,15 @@ __global__ __launch_bounds__(64 * kMidWaves, 2) void gemm_mid_kernel(GemmArgs a,
   // the range load zeros and add nothing.
   const int bsteps = a.gs_stride / 16;
   const int st_lo = split * bsteps / S, st_hi = (split + 1) * bsteps / S;
-  const int st_pro = BOOK == kAffine ? min(st_hi, st_lo + kMidBiasPro) : st_lo;
-  MidBias bias;
+  const int st_pro = BOOK == kAffine ? min(st_hi, st_lo + kBiasSrcPro) : st_lo;
+  BiasSrc bias;
   bias.rgs = make_rsrc(a.gs, BOOK == kAffine ? (uint32_t)((size_t)a.M * a.gs_stride * 2) : 0u);
   bias.rsb = make_rsrc(src.s, src.srange);
   bias.svoff = src.svoff;
   bias.M = a.M; bias.gs_stride = a.gs_stride; bias.G4 = G4; bias.m0 = m0; bias.c32 = c32; bias.h = h;
   if constexpr (BOOK == kAffine) {
-    u32x4 bv[kMidBiasPro], ba[kMidBiasPro][MT];
-    mid_bias_load<SD, MT>(bias, bv, ba, st_lo, st_pro);
+    u32x4 bv[kBiasSrcPro], ba[kBiasSrcPro][MT];
+    bias_load<SD, MT>(bias, bv, ba, st_lo, st_pro);
     __builtin_amdgcn_sched_barrier(0);        // requested before the ring: they complete first
 #pragma unroll
     for (int s = 0; s < R; ++s) {
@@ -216,7 +167,7 @@ __global__ __launch_bounds__(64 * kMidWaves, 2) void gemm_mid_kernel(GemmArgs a,
       mid_weights<BOOK>(src, s, wq[s], sp[s]);
     }
     __builtin_amdgcn_sched_barrier(0);
-    mid_bias_mul<SD, MT>(bv, ba, h, acc);
+    bias_mul<SD, MT>(bv, ba, h, acc);
   } else {
 #pragma unroll
     for (int s = 0; s < R; ++s) {
@@ -329,10 +280,10 @@ __global__ __launch_bounds__(64 * kMidWaves, 2) void gemm_mid_kernel(GemmArgs a,
         const int fm = MT == 1 ? 0 : c;
         acc[fm][v] = __builtin_fmaf(sc[c], pp[1][c][v], acc[fm][v]);
       }
-    for (int st0 = st_pro; st0 < st_hi; st0 += kMidBiasChunk) {
-      u32x4 bv[kMidBiasChunk], ba[kMidBiasChunk][MT];
-      mid_bias_load<SD, MT>(bias, bv, ba, st0, st_hi);
-      mid_bias_mul<SD, MT>(bv, ba, h, acc);
+    for (int st0 = st_pro; st0 < st_hi; st0 += kBiasSrcChunk) {
+      u32x4 bv[kBiasSrcChunk], ba[kBiasSrcChunk][MT];
+      bias_load<SD, MT>(bias, bv, ba, st0, st_hi);
+      bias_mul<SD, MT>(bv, ba, h, acc);
     }
   }
   __builtin_amdgcn_s_waitcnt(0);              // no LDS-DMA outlives the workgroup's LDS

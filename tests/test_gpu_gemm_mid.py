@@ -1,6 +1,7 @@
-"""The prefill kernel for calls with few output tiles (gemm_mid.hip) against the one for many
-(gemm.hip): a row has the same bits whichever of them its call runs, at the edges of the row
-tiles (32 and 64 rows), with a ragged N (tiles of 16, 32 and 128 features cut), an odd number
+"""The prefill kernels for calls with few output tiles (gemm_mid.hip, and gemm_few.hip for a few
+rows) against the one for many (gemm.hip): a row has the same bits whichever of them its call
+runs, at the edges of the row tiles (8, 16, 32 and 64 rows) and of the few-row kernel's range
+(256 tiles of 32 x 32), with a ragged N (tiles of 16, 32 and 128 features cut), an odd number
 of groups (the last pair half empty), more bias steps than run ahead of the K loop, a split K,
 bf16 scales, ACCUM and every native codebook; and the rows match the fp64 product."""
 
@@ -15,8 +16,9 @@ TOL = 1e-3
 
 # K, N, scales, rows of the call whose 128 x 256 tiles fill the chip (gemm.hip); the third
 # splits K in two
-SHAPES = [(1024, 1000, "f16", 16384), (1088, 300, "bf16", 16384), (8192, 1000, "f16", 4352), (320, 1500, "bf16", 16384)]
-ROWS = [9, 31, 32, 33, 64, 65, 127, 300]
+SHAPES = [(1024, 1000, "f16", 16384), (1088, 300, "bf16", 16384), (8192, 1000, "f16", 4352), (320, 1500, "bf16", 16384),
+          (320, 40, "f16", 40000), (9216, 4200, "bf16", 4352)]
+ROWS = [9, 16, 17, 31, 32, 33, 64, 65, 127, 224, 257, 300]
 
 
 @pytest.mark.parametrize("K,N,sd,M", SHAPES)
