@@ -30,8 +30,8 @@ namespace rlq {
 constexpr int kMidWaves = 4;             // (two per workgroup measured the same on small grids, up to 1.6 times slower on full ones)
 constexpr int kMidCols = 32 * kMidWaves; // features of a workgroup
 constexpr int kMidRow = 256;             // LDS bytes of one row of a stage: one pair of groups, 128 fp16
-constexpr int kBiasSrcPro = 11;          // bias steps before the K loop, as gemm4_kernel runs them
-constexpr int kBiasSrcChunk = 8;         // bias steps loaded at a time after it
+constexpr int kMidBiasPro = 11;          // bias steps before the K loop, as gemm4_kernel runs them
+constexpr int kMidBiasChunk = 8;         // bias steps loaded at a time after it
 
 template <int MT> constexpr int mid_stage_bytes() { return 32 * MT * kMidRow; }
 
@@ -151,14 +151,14 @@ __global__ __launch_bounds__(64 * kMidWaves, 2) void gemm_mid_kernel(GemmArgs a,
   // the range load zeros and add nothing.
   const int bsteps = a.gs_stride / 16;
   const int st_lo = split * bsteps / S, st_hi = (split + 1) * bsteps / S;
-  const int st_pro = BOOK == kAffine ? min(st_hi, st_lo + kBiasSrcPro) : st_lo;
+  const int st_pro = BOOK == kAffine ? min(st_hi, st_lo + kMidBiasPro) : st_lo;
   BiasSrc bias;
   bias.rgs = make_rsrc(a.gs, BOOK == kAffine ? (uint32_t)((size_t)a.M * a.gs_stride * 2) : 0u);
   bias.rsb = make_rsrc(src.s, src.srange);
   bias.svoff = src.svoff;
   bias.M = a.M; bias.gs_stride = a.gs_stride; bias.G4 = G4; bias.m0 = m0; bias.c32 = c32; bias.h = h;
   if constexpr (BOOK == kAffine) {
-    u32x4 bv[kBiasSrcPro], ba[kBiasSrcPro][MT];
+    u32x4 bv[kMidBiasPro], ba[kMidBiasPro][MT];
     bias_load<SD, MT>(bias, bv, ba, st_lo, st_pro);
     __builtin_amdgcn_sched_barrier(0);        // requested before the ring: they complete first
 #pragma unroll
@@ -280,8 +280,8 @@ __global__ __launch_bounds__(64 * kMidWaves, 2) void gemm_mid_kernel(GemmArgs a,
         const int fm = MT == 1 ? 0 : c;
         acc[fm][v] = __builtin_fmaf(sc[c], pp[1][c][v], acc[fm][v]);
       }
-    for (int st0 = st_pro; st0 < st_hi; st0 += kBiasSrcChunk) {
-      u32x4 bv[kBiasSrcChunk], ba[kBiasSrcChunk][MT];
+    for (int st0 = st_pro; st0 < st_hi; st0 += kMidBiasChunk) {
+      u32x4 bv[kMidBiasChunk], ba[kMidBiasChunk][MT];
       bias_load<SD, MT>(bias, bv, ba, st0, st_hi);
       bias_mul<SD, MT>(bv, ba, h, acc);
     }
