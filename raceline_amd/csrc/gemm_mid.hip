@@ -45,21 +45,22 @@ struct MidSrc {
   int K, pb, n, wave, c0;       // the split's first pair and its pairs; the logical chunk of DMA 0
 };
 
-// The loads of pair q (counted from the split's first): its codes and scale words into
-// registers (mid_weights), its activation rows into stage s of the ring (mid_rows).
-// Straight-line, the same number for every pair, so that the waits count them: past the last
+// One load of pair q (counted from the split's first): part 0 or 1 of its codes, part 2 its
+// scale words, into registers (mid_weights), or one of the wave's DMAs of its activation
+// rows into stage s of the ring (mid_rows). Every pair makes the same number of loads, so that
+// the waits count them: past the last
 // pair the descriptors are empty, and the loads touch no memory. The pair's offset goes in
 // the scalar operand, which the range check does not see: it stays inside a tile (p < 2 G4)
 // and, for inputs below K, inside a row; where the last pair holds one group (an odd number
 // of groups), the chunks of the other take an offset past every range and read zeros.
-template <int BOOK, int DMA>
-__device__ __forceinline__ void mid_weights(const MidSrc<DMA> &src, int q, u32x4 (&wq)[2], uint64_t &sp) {
+template <int DMA>
+__device__ __forceinline__ void mid_weights(const MidSrc<DMA> &src, int part, int q, u32x4 (&wq)[2], uint64_t &sp) {
   const bool live = q < src.n;
   const int p = live ? src.pb + q : 0;
-  const __amdgpu_buffer_rsrc_t rw = make_rsrc(src.w, live ? src.wrange : 0u);
-  wq[0] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, src.wvoff, p * 1024, 0));
-  wq[1] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, src.wvoff + 512u, p * 1024, 0));
-  if constexpr (BOOK == kAffine) {
+  if (part < 2) {
+    const __amdgpu_buffer_rsrc_t rw = make_rsrc(src.w, live ? src.wrange : 0u);
+    wq[part] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, src.wvoff + 512u * part, p * 1024, 0));
+  } else {
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(src.s, live ? src.srange : 0u);
     sp = __builtin_bit_cast(uint64_t,
                             __builtin_amdgcn_raw_buffer_load_b64(rs, src.svoff, (p >> 1) * 256 + 8 * (p & 1), 0));
@@ -67,15 +68,14 @@ __device__ __forceinline__ void mid_weights(const MidSrc<DMA> &src, int q, u32x4
 }
 
 template <int MT, int DMA>
-__device__ __forceinline__ void mid_rows(const MidSrc<DMA> &src, unsigned char *lds, int s, int q) {
+__device__ __forceinline__ void mid_rows(const MidSrc<DMA> &src, unsigned char *lds, int s, int q, int i) {
   const bool live = q < src.n;
   const int p = live ? src.pb + q : 0;
   const __amdgpu_buffer_rsrc_t rx = make_rsrc(src.x, live ? src.xrange : 0u);
   const bool tail = 128 * (p + 1) > src.K;
-#pragma unroll
-  for (int i = 0; i < DMA; ++i)   // the rows of DMA i are 16 i past DMA 0's: the same logical chunk
-    dma16(rx, lds, s * mid_stage_bytes<MT>() + (src.wave + kMidWaves * i) * 1024,
-          tail && (src.c0 & 8) ? kFarOffset : src.aoff[i], 256 * p);
+  // the rows of DMA i are 16 i past DMA 0's: the same logical chunk
+  dma16(rx, lds, s * mid_stage_bytes<MT>() + (src.wave + kMidWaves * i) * 1024,
+        tail && (src.c0 & 8) ? kFarOffset : src.aoff[i], 256 * p);
 }
 
 template <int BOOK, int SD, int MT, int R>
@@ -83,7 +83,8 @@ __global__ __launch_bounds__(64 * kMidWaves, 2) void gemm_mid_kernel(GemmArgs a,
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   constexpr int kStage = mid_stage_bytes<MT>();
   constexpr int kDma = 8 * MT / kMidWaves;                        // activation LDS-DMAs per wave and pair
-  constexpr int kLoads = kDma + 2 + (BOOK == kAffine ? 1 : 0);   // vector memory loads per wave and pair
+  constexpr int kParts = BOOK == kAffine ? 3 : 2;         // weight loads per wave and pair
+  constexpr int kLoads = kDma + kParts;                   // vector memory loads per wave and pair
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int G = a.K / kGroup, G4 = quads_of(a.K), GP = 2 * G4;
@@ -157,23 +158,28 @@ __global__ __launch_bounds__(64 * kMidWaves, 2) void gemm_mid_kernel(GemmArgs a,
   bias.rsb = make_rsrc(src.s, src.srange);
   bias.svoff = src.svoff;
   bias.M = a.M; bias.gs_stride = a.gs_stride; bias.G4 = G4; bias.m0 = m0; bias.c32 = c32; bias.h = h;
+  // the first R pairs; the weights of the last of them follow in the first round
+  auto fill = [&]() {
+#pragma unroll
+    for (int s = 0; s < R; ++s) {
+#pragma unroll
+      for (int i = 0; i < kDma; ++i) mid_rows<MT>(src, lds, s, s, i);
+      if (s + 1 < R) {
+#pragma unroll
+        for (int i = 0; i < kParts; ++i) mid_weights(src, i, s, wq[s], sp[s]);
+      }
+      __builtin_amdgcn_sched_barrier(0);      // in the order they are used
+    }
+  };
   if constexpr (BOOK == kAffine) {
     u32x4 bv[kMidBiasPro], ba[kMidBiasPro][MT];
     bias_load<SD, MT>(bias, bv, ba, st_lo, st_pro);
     __builtin_amdgcn_sched_barrier(0);        // requested before the ring: they complete first
-#pragma unroll
-    for (int s = 0; s < R; ++s) {
-      mid_rows<MT>(src, lds, s, s);
-      mid_weights<BOOK>(src, s, wq[s], sp[s]);
-    }
+    fill();
     __builtin_amdgcn_sched_barrier(0);
     bias_mul<SD, MT>(bv, ba, h, acc);
   } else {
-#pragma unroll
-    for (int s = 0; s < R; ++s) {
-      mid_rows<MT>(src, lds, s, s);
-      mid_weights<BOOK>(src, s, wq[s], sp[s]);
-    }
+    fill();
   }
   __builtin_amdgcn_s_waitcnt(waitcnt_vmcnt((R - 1) * kLoads));   // pair 0 has landed for this wave
   asm volatile("s_barrier" ::: "memory");   // and for every wave
@@ -206,22 +212,22 @@ __global__ __launch_bounds__(64 * kMidWaves, 2) void gemm_mid_kernel(GemmArgs a,
 
   // PAR: which half of the double buffers the round uses; gg: its group (MT = 2)
   auto round = [&](auto slot_c, auto par_c, int gg, int q) {
-    constexpr int SL = decltype(slot_c)::value, NX = (SL + 1) % R, PAR = decltype(par_c)::value;
+    constexpr int SL = decltype(slot_c)::value, NX = (SL + 1) % R, PV = (SL + R - 1) % R, PAR = decltype(par_c)::value;
     const bool last = MT == 1 || gg == 1;             // the pair's last round: the next one reads the next stage
     float scn[2] = {0.0f, 0.0f};
     if constexpr (BOOK == kAffine) {
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
         scn[c] = scale_f32<SD>((uint16_t)(sp[SL] >> (32 * (MT == 1 ? c : gg)))) * kTwo24;
-        asm volatile("" : "+v"(scn[c]));              // taken now: the slot's next load is issued below
+        asm volatile("" : "+v"(scn[c]));              // taken now: the slot's next load is issued in the next round
       }
     }
     if (last) {
       // the pair's fragments are all in registers: its stage is free once every wave is
       // here, and pair q + 1's rows have landed when each wave's own part has
-      __builtin_amdgcn_s_waitcnt(0x0070 | (waitcnt_vmcnt((R - 2) * kLoads + kLoads - kDma) & 0xC00F));   // and lgkmcnt(0)
+      // (MT = 2: the weights of this pair's first round have gone out since)
+      __builtin_amdgcn_s_waitcnt(0x0070 | (waitcnt_vmcnt((R - 2) * kLoads + (MT == 1 ? 0 : kParts)) & 0xC00F));   // and lgkmcnt(0)
       asm volatile("s_barrier" ::: "memory");
-      mid_rows<MT>(src, lds, SL, q + R);
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -231,6 +237,14 @@ __global__ __launch_bounds__(64 * kMidWaves, 2) void gemm_mid_kernel(GemmArgs a,
 #pragma unroll
         for (int e = 2 * j; e < 2 * j + 2; ++e) fr[PAR ^ 1][e] = last ? step_frag(NX, 0, e) : step_frag(SL, 1, e);
       }
+      // The loads go out a step or two apart: all of a pair's at once, right after the
+      // barrier, queued behind those of the workgroup's other waves (about 60 cycles each).
+      // Weights: the slot of the pair before, whose codes are all used; rows: this pair's
+      // stage. The last load of a pair is a DMA (the wait above counts on it).
+      if (MT == 1 || gg == 0) {
+        if ((j & 1) && j / 2 < kParts) mid_weights(src, j / 2, q - 1 + R, wq[PV], sp[PV]);
+      }
+      if (last && (MT == 1 ? j == 2 || j == 6 : (j & 1) == 0)) mid_rows<MT>(src, lds, SL, q + R, MT == 1 ? j / 4 : j / 2);
       const half8 b = bf[(MT == 1 ? j : i) & 1];
       if (MT == 1 || c == 1) {                        // the next step's codes (MT = 2: both chains share them)
         const int nj = j + 1, slot = ((MT == 1 ? nj : i + 1)) & 1;
@@ -251,7 +265,6 @@ __global__ __launch_bounds__(64 * kMidWaves, 2) void gemm_mid_kernel(GemmArgs a,
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (last) mid_weights<BOOK>(src, q + R, wq[SL], sp[SL]);   // the slot's codes are all used
     sc[0] = scn[0];
     sc[1] = scn[1];
   };
