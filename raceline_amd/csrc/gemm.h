@@ -40,7 +40,7 @@ int run_gemm4(int book, const _Float16 *x, int x_stride, int M, int K, int N, co
 // The kernel for calls with too few 128 x 256 tiles (gemm_mid.hip): gemm_mid_tiles gives the
 // 32-row tiles (1 or 2) of its workgroups' rows, or 0 where gemm4_kernel takes the call. Both
 // kernels give the same bits.
-int gemm_mid_tiles(int M, int K, int N, int S);
+int gemm_mid_tiles(int book, int M, int K, int N, int S);
 int launch_gemm_mid(int book, int sd, int mt, const GemmArgs &a, int S, int accum, hipStream_t st);
 
 // The affine kernel for a few rows (gemm_few.hip), the same bits again, and whether it takes a

@@ -813,7 +813,7 @@ int run_gemm4(int book, const _Float16 *x, int x_stride, int M, int K, int N, co
       if (int rc = launch_gemm_few(sd, c, S, accum, st)) return rc;
       continue;
     }
-    if (const int mt = gemm_mid_tiles(c.M, K, N, S)) {   // too few of this kernel's tiles to fill the chip
+    if (const int mt = gemm_mid_tiles(book, c.M, K, N, S)) {   // too few of this kernel's tiles to fill the chip
       if (int rc = launch_gemm_mid(book, sd, mt, c, S, accum, st)) return rc;
       continue;
     }

@@ -419,28 +419,34 @@ static int launch_mid_rows(int mt, const GemmArgs &a, int S, int accum, hipStrea
   return mt == 1 ? launch_mid<BOOK, SD, 1>(a, S, accum, st) : launch_mid<BOOK, SD, 2>(a, S, accum, st);
 }
 
-// Which kernel and tile take a call: the one of three estimated fastest, each as (rounds of
-// the chip) x (group pairs per workgroup) x (time of a pair), from launches timed with their
-// prep pass on 9B and 27B projections (K 4096 .. 17408, N 4096 .. 34816) at M = 16 .. 512:
-//  - this kernel, 32 rows x 128 features: 0.40 us per pair and wave of each SIMD. A wave
-//    alone on its SIMD is bound by its own instruction issue (147 issue slots of 4 cycles
-//    per pair, 62% of its cycles), and two resident ones together take as long as one after
-//    the other: K = 12288, N = 4096 42 us at M = 16, 44 at 64, 69 at 300 (from 153, 156, 163
-//    with gemm4_kernel, whose 16 .. 48 workgroups leave the chip empty);
-//  - 64 rows x 128 features: 0.63 us (each code converted once for two row tiles);
-//  - gemm4_kernel, 128 x 256: 1.5 us with the chip nearly empty to 2.2 us full (the stage
-//    loads and the clock of a full chip).
-// At K = 5120, N = 34816: M = 16 38 us (64 x 128: 47, gemm4 74), M = 128 83 (82, 80),
-// M = 300 175 (150, 158).
-int gemm_mid_tiles(int M, int K, int N, int S) {
+// Which kernel and tile take a call: the one of three estimated fastest (32 or 64 rows x 128
+// features here, gemm4_kernel's 128 x 256), each as
+//   once + group pairs per workgroup x (per_round x rounds of the chip + per_fill x units / units of a round),
+// in us, fitted to launches timed with their prep pass on 9B and 27B projections (K 4096 ..
+// 12288, N 4096 .. 34816) at M = 16 .. 1024. A wave here is bound by its own instruction
+// issue, and two resident on a SIMD take about as long as one after the other, so the rounds
+// count; how full they are costs memory time and clock. The books differ in what a code
+// costs to convert (4 operations for eight fp4 codes, 14 for eight int15 ones, shared by two row
+// tiles at 64 rows), the affine one in its scale FMAs. Against the fastest of the three at 65
+// shapes a book, the choice loses 0.3% on average and 4% at most (affine), 0.1% and 4%
+// (integer books), 0.2% and 6% (fp4); one set of constants for all books lost up to 12% and
+// 30%: int15 K = 5120, N = 34816 at M = 48 took the 32-row tile, 49.4 us, for the 64-row
+// tile's 38.1; affine K = 4096, N = 24576 at M = 256 the 64-row tile, 67.8, for gemm4's 60.4.
+struct MidCost { double once, per_round, per_fill; };
+constexpr MidCost kCostAffine[3] = {{5.7, 1.48, 0.38}, {10.5, 0.25, 0.10}, {13.5, 0.41, 0.15}};   // gemm4, 32 rows, 64 rows
+constexpr MidCost kCostInt[3] = {{3.4, 1.33, 0.41}, {7.4, 0.35, 0.0}, {6.5, 0.43, 0.07}};
+constexpr MidCost kCostFp4[3] = {{8.0, 1.5, 0.7}, {6.0, 0.40, 0.0}, {6.0, 0.63, 0.0}};
+
+int gemm_mid_tiles(int book, int M, int K, int N, int S) {
+  const MidCost *cost = book == kAffine ? kCostAffine : book == kFp4 ? kCostFp4 : kCostInt;
   const double pairs = ((K / kGroup + 1) / 2 + S - 1) / S;
-  auto rounds = [](long long units, int per) { return (double)((units + per - 1) / per); };
+  auto time = [&](const MidCost &c, long long units, int per) {
+    return c.once + pairs * (c.per_round * (double)((units + per - 1) / per) + c.per_fill * (double)units / per);
+  };
   const long long nt = (N + 31) / 32;
-  const double t1 = 6 + pairs * 0.40 * rounds(nt * ((M + 31) / 32) * S, 1024);
-  const double t2 = 6 + pairs * 0.63 * rounds(nt * ((M + 63) / 64) * S, 1024);
-  const long long wg4 = (long long)((N + 255) / 256) * ((M + 127) / 128) * S;
-  const double r4 = rounds(wg4, 256);
-  const double t4 = 8 + pairs * r4 * (1.5 + 0.7 * (double)wg4 / (256 * r4));
+  const double t4 = time(cost[0], (long long)((N + 255) / 256) * ((M + 127) / 128) * S, 256);
+  const double t1 = time(cost[1], nt * ((M + 31) / 32) * S, 1024);
+  const double t2 = time(cost[2], nt * ((M + 63) / 64) * S, 1024);
   // a split call's tiles count their arrivals in the workspace's counters
   auto fits = [&](int mt) { return S == 1 || (long long)((M + 32 * mt - 1) / (32 * mt)) * ((N + kMidCols - 1) / kMidCols) <= kGemmMaxCounters; };
   if (t1 <= t2 && t1 < t4 && fits(1)) return 1;
