@@ -426,7 +426,7 @@ static int launch_mid_rows(int mt, const GemmArgs &a, int S, int accum, hipStrea
 // 12288, N 4096 .. 34816) at M = 16 .. 1024. A wave here is bound by its own instruction
 // issue, and two resident on a SIMD take about as long as one after the other, so the rounds
 // count; how full they are costs memory time and clock. The books differ in what a code
-// costs to convert (4 operations for eight fp4 codes, 14 for eight int15 ones, shared by two row
+// costs to convert (4 operations for eight fp4 codes, 13 for eight integer ones, shared by two row
 // tiles at 64 rows), the affine one in its scale FMAs. Against the fastest of the three at 65
 // shapes a book, the choice loses 0.3% on average and 4% at most (affine), 0.1% and 4%
 // (integer books), 0.2% and 6% (fp4); one set of constants for all books lost up to 12% and

@@ -63,34 +63,6 @@ __device__ __forceinline__ float scale_f32(uint16_t bits) {
   }
 }
 
-// Two fp16 values 1024 + a, 1024 + b (a, b < 1024 integers, as the low bits of each half
-// over the exponent pattern 0x6400) minus (1024 + OFF): exactly a - OFF and b - OFF, as
-// normal fp16 numbers. (Codes go to the matrix cores as normal numbers: the f16 MFMA of
-// gfx950 sums products of subnormal operands with about five bits less precision than
-// normal ones.)
-template <int OFF = 0>
-__device__ __forceinline__ uint32_t magic_pair_to_f16(uint32_t bits) {
-  typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-  const half2v m = {(_Float16)(-1024.0f - OFF), (_Float16)(-1024.0f - OFF)};
-  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, bits | 0x64006400u) + m);
-}
-
-// Eight 4-bit codes of one uint32 (element e at bits 4e, tools/convert.py:82-89) -> eight
-// fp16 operands q0 - OFF .. q7 - OFF, in element order: two masks, one shift, four byte
-// permutes, four or + packed-add pairs.
-template <int OFF = 0>
-__device__ __forceinline__ half8 nib8_to_half8(uint32_t u) {
-  const uint32_t lo = u & 0x0F0F0F0Fu;         // bytes: q0 q2 q4 q6
-  const uint32_t hi = (u >> 4) & 0x0F0F0F0Fu;  // bytes: q1 q3 q5 q7
-  // perm(S0=hi, S1=lo, sel): selector 0..3 picks bytes of lo, 4..7 bytes of hi, 0x0C a zero byte.
-  u32x4 d;
-  d[0] = magic_pair_to_f16<OFF>(__builtin_amdgcn_perm(hi, lo, 0x0C040C00u));  // (q0, q1)
-  d[1] = magic_pair_to_f16<OFF>(__builtin_amdgcn_perm(hi, lo, 0x0C050C01u));  // (q2, q3)
-  d[2] = magic_pair_to_f16<OFF>(__builtin_amdgcn_perm(hi, lo, 0x0C060C02u));  // (q4, q5)
-  d[3] = magic_pair_to_f16<OFF>(__builtin_amdgcn_perm(hi, lo, 0x0C070C03u));  // (q6, q7)
-  return __builtin_bit_cast(half8, d);
-}
-
 // Codebooks of the native format (tools/quantlib.py:23-28). kInt15: two's complement
 // -8 .. 7; kInt16: the same plus 0.5 (applied as 0.5 * sum of the activations, as
 // kernels/linear.metal:128-129,171-172 do); kFp4: e2m1, sign in bit 3.
@@ -99,7 +71,13 @@ enum Book { kAffine = 0, kInt15 = 1, kInt16 = 2, kFp4 = 3 };
 // Eight native codes -> their codebook values as fp16, in element order. kFp4: the
 // hardware's e2m1 -> fp16 conversion, two codes (one byte, low nibble first) per
 // instruction; with scale 1 every value is exact: 0, 0.5, 1, 1.5, 2, 3, 4, 6, signed by
-// bit 3 (the same bits as a table lookup of the codebook).
+// bit 3 (the same bits as a table lookup of the codebook). The integer books: with
+// q' = q ^ 8, a byte permute puts the byte of two codes into both halves under the exponent
+// pattern 0x64, a mask leaves 1024 + q'0 and 1024 + 16 q'1, and one packed fused multiply-add
+// by (1, 1/16) gives q' - 8, the signed value, exactly. (Codes go to the matrix cores as
+// normal numbers: the f16 MFMA of gfx950 sums products of subnormal operands with about five
+// bits less precision.) Thirteen operations for eight codes; sixteen, with the codes of a pair
+// gathered from two masked words, took K = 12288, N = 4096 at 16 rows 45.2 us instead of 40.1.
 template <int BOOK>
 __device__ __forceinline__ half8 native8_to_half8(uint32_t u) {
   if constexpr (BOOK == kFp4) {
@@ -110,7 +88,15 @@ __device__ __forceinline__ half8 native8_to_half8(uint32_t u) {
     d[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(u, 1.0f, 3));
     return __builtin_bit_cast(half8, d);
   } else {
-    return nib8_to_half8<8>(u ^ 0x88888888u);   // (q ^ 8) - 8: the signed value
+    typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+    const half2v mul = {(_Float16)1.0f, (_Float16)0.0625f}, off = {(_Float16)-1032.0f, (_Float16)-72.0f};
+    const uint32_t v = u ^ 0x88888888u;
+    auto two = [&](uint32_t sel) {   // selector 4 .. 7: a byte of v, 0: 0x64
+      const uint32_t bits = __builtin_amdgcn_perm(v, 0x64646464u, sel) & 0x64F0640Fu;
+      return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, bits) * mul + off);
+    };
+    const u32x4 d = {two(0x00040004u), two(0x00050005u), two(0x00060006u), two(0x00070007u)};
+    return __builtin_bit_cast(half8, d);
   }
 }
 
@@ -121,7 +107,7 @@ __device__ __forceinline__ half8 native8_to_half8(uint32_t u) {
 // two normal fp16 numbers over the exponent pattern 0x6400, as 1024 + q', and codes 1 and 5
 // (3 and 7) as 1024 + 16 q'; one packed add, or fused multiply-add, per pair then gives
 // q' - 8, the signed value, exactly: (1024 + q') - 1032 and (1024 + 16 q') / 16 - 72. Ten
-// operations for eight codes, against sixteen in element order.
+// operations for eight codes, against thirteen in element order.
 template <int BOOK>
 __device__ __forceinline__ half8 native8_operand(uint32_t u) {
   if constexpr (BOOK == kFp4) {
