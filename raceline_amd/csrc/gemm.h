@@ -27,7 +27,7 @@ struct GemmArgs {
 constexpr int kGemmMaxCounters = 1024;
 
 // Bytes of workspace run_gemm4 needs (affine: the prepped activations and the split group
-// sums; kInt16: group and row sums; a shape whose K is split: the partial products).
+// sums; kInt16: row sums; a shape whose K is split: the partial products).
 size_t gemm4_workspace(int book, int M, int K, int N);
 
 // codes, sbq: the two sections of a packed matrix (q4_tile.h), or of rows [r0, r0 + N) of a
@@ -49,7 +49,6 @@ bool gemm_few_fits(int M, int N, int S);
 int launch_gemm_few(int sd, const GemmArgs &a, int S, int accum, hipStream_t st);
 
 // defined in linear.hip
-void launch_group_sums(const _Float16 *x, int x_stride, int M, int K, float *gsT, int m_pad, hipStream_t st);
-void launch_row_sums(const float *gsT, int G, int m_pad, int M, float *asum, hipStream_t st);
+void launch_row_sums(const _Float16 *x, int x_stride, int M, int K, float *asum, hipStream_t st);
 
 }  // namespace rlq

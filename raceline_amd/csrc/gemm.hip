@@ -718,7 +718,7 @@ static size_t books_workspace(int book, int M, int K) {
   if (book == kAffine)   // the group-sum pieces sized for bf16 biases, the larger of the two
     return ((size_t)M * K * 2 + 255) / 256 * 256 + ((size_t)M * gs_stride_of(G, 1) * 2 + 255) / 256 * 256 +
            ((size_t)M * sizeof(float) + 255) / 256 * 256;
-  if (book == kInt16) return ((size_t)(G + 1) * ((M + 127) / 128 * 128) * sizeof(float) + 255) / 256 * 256;
+  if (book == kInt16) return ((size_t)M * sizeof(float) + 255) / 256 * 256;
   return 0;
 }
 
@@ -785,11 +785,9 @@ int run_gemm4(int book, const _Float16 *x, int x_stride, int M, int K, int N, co
   } else {
     a.x = x; a.x_stride = x_stride;
     if (book == kInt16) {
-      const int m_pad = (M + 127) / 128 * 128;
-      float *gsT = static_cast<float *>(ws);
-      float *asum = gsT + (size_t)G * m_pad;
-      launch_group_sums(x, x_stride, M, K, gsT, m_pad, st);
-      launch_row_sums(gsT, G, m_pad, M, asum, st);
+      float *asum = static_cast<float *>(ws);
+      launch_row_sums(x, x_stride, M, K, asum, st);
+      RLQ_HIP(hipGetLastError());
       a.asum = asum;
     }
   }

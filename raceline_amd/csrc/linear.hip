@@ -782,14 +782,10 @@ int linear_packed(int kernel, int book, const _Float16 *x, int x_stride, int M, 
 
 // ================================================================== group sums
 
-// gsum[m][g] and/or its transpose gsT[g][m_pad], summed sequentially in fp32 as
-// group_sums does (kernels/linear.metal:34-45).
-__global__ void group_sums_kernel(const _Float16 *x, int x_stride, int M, int K, float *gsum, float *gsT, int m_pad) {
-  const int G = K / kGroup;
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= M * G) return;
-  const int m = idx / G, g = idx - m * G;
-  const half8 *xp = reinterpret_cast<const half8 *>(x + (size_t)m * x_stride + (size_t)g * kGroup);
+// A group's 64 activations summed sequentially in fp32, as group_sums does
+// (kernels/linear.metal:34-45).
+__device__ __forceinline__ float group_sum(const _Float16 *x) {
+  const half8 *xp = reinterpret_cast<const half8 *>(x);
   float sum = 0.0f;
 #pragma unroll
   for (int c = 0; c < 8; ++c) {
@@ -797,27 +793,50 @@ __global__ void group_sums_kernel(const _Float16 *x, int x_stride, int M, int K,
 #pragma unroll
     for (int e = 0; e < 8; ++e) sum += static_cast<float>(v[e]);
   }
-  if (gsum) gsum[(size_t)m * G + g] = sum;
-  if (gsT) gsT[(size_t)g * m_pad + m] = sum;
+  return sum;
 }
 
-// asum[m] = sum over g of gsT[g][m], in order: the activation row sums the half-step
-// codebook needs.
-__global__ void row_sums_kernel(const float *gsT, int G, int m_pad, int M, float *asum) {
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= M) return;
-  float s = 0.0f;
-  for (int g = 0; g < G; ++g) s += gsT[(size_t)g * m_pad + m];
-  asum[m] = s;
-}
-
-void launch_group_sums(const _Float16 *x, int x_stride, int M, int K, float *gsT, int m_pad, hipStream_t st) {
+// gsum[m][g]
+__global__ void group_sums_kernel(const _Float16 *x, int x_stride, int M, int K, float *gsum) {
   const int G = K / kGroup;
-  group_sums_kernel<<<(M * G + 255) / 256, 256, 0, st>>>(x, x_stride, M, K, nullptr, gsT, m_pad);
+  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= M * G) return;
+  const int m = idx / G, g = idx - m * G;
+  gsum[(size_t)m * G + g] = group_sum(x + (size_t)m * x_stride + (size_t)g * kGroup);
 }
 
-void launch_row_sums(const float *gsT, int G, int m_pad, int M, float *asum, hipStream_t st) {
-  row_sums_kernel<<<(M + 255) / 256, 256, 0, st>>>(gsT, G, m_pad, M, asum);
+// asum[m] = the sum over a row's groups, in order, of their sums (each summed in order too):
+// the activation row sums the half-step codebook needs. One workgroup per row: a thread sums
+// a group, one thread adds the group sums from the LDS. Bound by its launch and that chain
+// of adds (latency): with a launch for the group sums and one thread per row adding them from
+// memory, int16 calls of 16 rows
+// took 18 us longer than int15 ones at K = 4096 and 47 at K = 12288, now 3.
+constexpr int kRowSumChunk = 1024;   // group sums in the LDS at a time
+__global__ void row_sums_kernel(const _Float16 *x, int x_stride, int K, float *asum) {
+  __shared__ f32x4 gs[kRowSumChunk / 4];
+  const int G = K / kGroup;
+  const _Float16 *row = x + (size_t)blockIdx.x * x_stride;
+  float s = 0.0f;
+  for (int g0 = 0; g0 < G; g0 += kRowSumChunk) {
+    const int n = min(kRowSumChunk, G - g0), n16 = (n + 15) / 16 * 16;
+    // (zeros up to a multiple of 16 change no sum: s is never -0)
+    for (int g = threadIdx.x; g < n16; g += blockDim.x)
+      reinterpret_cast<float *>(gs)[g] = g < n ? group_sum(row + (size_t)(g0 + g) * kGroup) : 0.0f;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int i = 0; i < n16 / 4; i += 4) {
+        const f32x4 v[4] = {gs[i], gs[i + 1], gs[i + 2], gs[i + 3]};
+#pragma unroll
+        for (int j = 0; j < 16; ++j) s += v[j >> 2][j & 3];
+      }
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) asum[blockIdx.x] = s;
+}
+
+void launch_row_sums(const _Float16 *x, int x_stride, int M, int K, float *asum, hipStream_t st) {
+  row_sums_kernel<<<M, std::min(256, (K / kGroup + 63) / 64 * 64), 0, st>>>(x, x_stride, K, asum);
 }
 
 static int check_linear_args(const char *fn, const void *x, int x_stride, int M, int K, int N, const void *packed,
@@ -987,7 +1006,7 @@ int rlq_group_sums(const void *x, int x_stride, int M, int K, float *gsum, void 
   RLQ_REQUIRE(x_stride >= K && x_stride % 8 == 0 && aligned(x, 16), "rlq_group_sums: x must be 16-byte aligned rows");
   const int G = K / kGroup;
   group_sums_kernel<<<(M * G + 255) / 256, 256, 0, static_cast<hipStream_t>(stream)>>>(
-      static_cast<const _Float16 *>(x), x_stride, M, K, gsum, nullptr, 0);
+      static_cast<const _Float16 *>(x), x_stride, M, K, gsum);
   RLQ_HIP(hipGetLastError());
   return 0;
 }

@@ -154,3 +154,29 @@ def test_raw_product(gpu, book, M, K, N):
     torch.cuda.synchronize()
     assert torch.equal(raw, unit)
     O.check_close(raw.cpu().numpy(), O.linear_native_f64(x, q, np.ones(N), book), TOL, f"raw {book} M={M}")
+
+
+@pytest.mark.parametrize("M,K,N", [(9, 64, 40), (33, 64 * 17, 100), (300, 64 * 65, 64), (10, 64 * 1025, 32)])
+def test_half_step_row_sums(gpu, M, K, N):
+    """int16 at prefill sizes is the int15 product plus half of each row's activation sum, as
+    one fma before the row scale (1 here): one group, a remainder of the 16 sums added at a
+    time, more groups than a wave has lanes: the same sums in the same order, so the same bits.
+    More than one LDS chunk of 1024 groups (K is split there and the fma comes before the
+    halves meet): the fp64 product."""
+    rng = np.random.default_rng(K)
+    q = rng.integers(0, 16, size=(N, K), dtype=np.uint8)
+    x = rng.standard_normal((M, K), dtype=np.float32).astype(np.float16)
+    one = np.ones(N, np.float32)
+    y16 = _run(gpu, x, _upload(q, one, "int16", gpu), kernel=2)
+    y15 = _run(gpu, x, _upload(q, one, "int15", gpu), kernel=2)
+    groups = np.zeros((M, K // 64), np.float32)
+    for e in range(64):
+        groups += x[:, e::64].astype(np.float32)
+    sums = np.zeros(M, np.float32)
+    for g in range(K // 64):
+        sums += groups[:, g]
+    if K > 64 * 1024:
+        O.check_close(y16, O.linear_native_f64(x, q, one, "int16"), TOL, "two chunks of group sums")
+        return
+    ref = y15.astype(np.float64) + 0.5 * sums.astype(np.float64)[:, None]
+    assert np.array_equal(y16, ref.astype(np.float32)), np.abs(y16 - ref).max()
