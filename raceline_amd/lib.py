@@ -113,6 +113,9 @@ def library_path() -> str:
                        "(or __graft_entry__.build()) or point RACELINE_LIB at it")
 
 
+_STATUS_FREE = ("rlq_abi_version", "rlq_set_fatal")   # int results that are no status
+
+
 @functools.lru_cache(maxsize=1)
 def load() -> ctypes.CDLL:
     lib = ctypes.CDLL(library_path())
@@ -120,6 +123,10 @@ def load() -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
+    # name -> (set_fatal, function, whether its int result is a status), kept on the library they
+    # belong to, so that a cleared cache of load() leaves none of an earlier library's
+    lib.entries = {name: (lib.rlq_set_fatal, getattr(lib, name), res is c_int and name not in _STATUS_FREE)
+                   for name, (res, _) in SIGNATURES.items()}
     return lib
 
 
@@ -127,21 +134,12 @@ class RlqError(RuntimeError):
     pass
 
 
-_STATUS_FREE = ("rlq_abi_version", "rlq_set_fatal")   # int results that are no status
-
-
-@functools.lru_cache(maxsize=None)
-def _entry(name: str):
-    """(set_fatal, function, whether its int result is a status) of one entry point."""
-    lib = load()
-    return lib.rlq_set_fatal, getattr(lib, name), SIGNATURES[name][0] is c_int and name not in _STATUS_FREE
-
-
 def call(name: str, *args):
     """Calls rlq_<name> in non-fatal mode and raises RlqError on a nonzero status."""
-    set_fatal, fn, status = _entry(name)
+    lib = load()
+    set_fatal, fn, status = lib.entries[name]
     set_fatal(0)
     rc = fn(*args)
     if status and rc != 0:
-        raise RlqError(f"{name}: {load().rlq_last_error().decode(errors='replace')}")
+        raise RlqError(f"{name}: {lib.rlq_last_error().decode(errors='replace')}")
     return rc

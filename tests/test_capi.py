@@ -121,3 +121,29 @@ def test_no_alloc_moe_refuses_sizes_past_its_scratch():
 def test_raw_native_product_refuses_the_half_step_book():
     with pytest.raises(lib.RlqError, match="no half step"):
         lib.call("rlq_linear_native_raw", 16, 64, 1, 64, 16, 16, 2, 16, 16, None, 0, None)
+
+
+def test_calls_follow_a_reloaded_library(tmp_path, monkeypatch):
+    """After load.cache_clear() (a library rebuilt in the same process) calls, their error mode
+    and their messages all come from the library that load() then gives, not from the one the
+    entry points were first bound to."""
+    import shutil
+
+    def failing():
+        lib.call("rlq_linear_affine", 16, 100, 1, 100, 10, 16, 0, 16, 10, 0, None, 0, None)
+
+    with pytest.raises(lib.RlqError, match="multiple of the group size"):
+        failing()
+    other = tmp_path / lib.LIB_NAME
+    shutil.copy(lib.library_path(), other)
+    monkeypatch.setenv("RACELINE_LIB", str(other))
+    lib.load.cache_clear()
+    try:
+        assert lib.load().rlq_last_error() == b""
+        with pytest.raises(lib.RlqError, match="multiple of the group size"):
+            failing()
+        assert lib.load().rlq_last_error().startswith(b"rlq_linear_affine")
+    finally:
+        monkeypatch.undo()
+        lib.load.cache_clear()
+        lib.load()
