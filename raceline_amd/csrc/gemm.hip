@@ -615,11 +615,11 @@ __global__ __launch_bounds__(kGThreads) void gemm4_kernel(GemmArgs a) {
     for (int v = 0; v < 16; ++v) {
       float val = acc[mt][v];
       if constexpr (BOOK == kAffine)   // undoes the prep's 2^e, exactly (the scale staged in the prologue)
-        val *= reinterpret_cast<const float *>(lds + kRscaleLds)[mt * 32 + 8 * (v >> 2) + 4 * h + (v & 3)];
+        val = mul_rounded(val, reinterpret_cast<const float *>(lds + kRscaleLds)[mt * 32 + 8 * (v >> 2) + 4 * h + (v & 3)]);
       if constexpr (BOOK == kInt16) {
         if (split == 0) val = __builtin_fmaf(0.5f, a.asum[min(m0 + mt * 32 + 8 * (v >> 2) + 4 * h + (v & 3), a.M - 1)], val);
       }
-      if constexpr (BOOK != kAffine) val *= rs_n;
+      if constexpr (BOOK != kAffine) val = mul_rounded(val, rs_n);
       if (acc_here) val = yv[v] + val;
       acc[mt][v] = val;
     }

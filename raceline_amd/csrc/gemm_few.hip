@@ -267,7 +267,7 @@ __global__ __launch_bounds__(kFewThreads, 3) void gemm_few_kernel(GemmArgs a, in
       float val = full[0][e];
 #pragma unroll
       for (int q = 1; q < 4; ++q) val = quarter == q ? full[0][4 * q + e] : val;
-      val *= rs[e];                                       // undoes the prep's 2^e, exactly
+      val = mul_rounded(val, rs[e]);                      // undoes the prep's 2^e, exactly
       if (acc_here) val = yv[e] + val;
       acc[e] = val;
     }

@@ -318,7 +318,7 @@ __global__ __launch_bounds__(64 * kMidWaves, 2) void gemm_mid_kernel(GemmArgs a,
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[mt][v] *= rs[mt][v];                   // undoes the prep's 2^e, exactly
+      for (int v = 0; v < 16; ++v) acc[mt][v] = mul_rounded(acc[mt][v], rs[mt][v]);   // undoes the prep's 2^e, exactly
   } else {
     const float rs_n = a.srow ? a.srow[nc] : 1.0f;                            // no row scales: the raw product
     if constexpr (BOOK == kInt16) {
@@ -333,7 +333,7 @@ __global__ __launch_bounds__(64 * kMidWaves, 2) void gemm_mid_kernel(GemmArgs a,
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[mt][v] *= rs_n;
+      for (int v = 0; v < 16; ++v) acc[mt][v] = mul_rounded(acc[mt][v], rs_n);
   }
   if (acc_here) {
     float yv[MT][16];

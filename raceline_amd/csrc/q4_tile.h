@@ -105,6 +105,16 @@ __device__ __forceinline__ u32x4 prep_x8(u32x4 p) {
 // definition for every kernel that applies it, so that they give the same bits
 __device__ __forceinline__ float silu(float v) { return v / (1.0f + expf(-v)); }
 
+// a * b, rounded to fp32 before what follows: without the barrier the compiler may fuse the
+// multiply into an add after it, in one kernel and not in another, and a row's bits would
+// depend on which of them its call runs. (Used outside the branch around the add: inside one
+// it keeps the compiler from making the branch a select.)
+__device__ __forceinline__ float mul_rounded(float a, float b) {
+  float v = a * b;
+  asm("" : "+v"(v));
+  return v;
+}
+
 // half(silu(g) * u) with the product rounded to fp32 and then to fp16, as the SwiGLU kernel
 // over fp32 gate/up rows computes it (moe_swiglu_kernel). The barrier keeps the compiler
 // from fusing the multiply into the conversion (v_fma_mix rounds once, which can differ in

@@ -180,3 +180,24 @@ def test_half_step_row_sums(gpu, M, K, N):
         return
     ref = y15.astype(np.float64) + 0.5 * sums.astype(np.float64)[:, None]
     assert np.array_equal(y16, ref.astype(np.float32)), np.abs(y16 - ref).max()
+
+
+@pytest.mark.parametrize("book", BOOKS)
+@pytest.mark.parametrize("M", [40, 300, 16384])   # short tiles; more of them; tiles that fill the chip
+def test_accumulating_adds_the_rounded_product(gpu, book, M):
+    """ACCUM at prefill sizes adds the product as the call without it writes it, rounded to fp32
+    after the row scale, whatever the row count: the same bits as the sum of the two."""
+    import torch
+
+    from raceline_amd import ops
+
+    K, N = 1088, 1000
+    rng = np.random.default_rng(M)
+    w = _upload(rng.integers(0, 16, size=(N, K), dtype=np.uint8), rng.uniform(0.002, 0.02, size=N), book, gpu)
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(M)
+    x = torch.randn((M, K), generator=gen, device=gpu).to(torch.float16)
+    h = torch.randn((M, N), generator=gen, device=gpu)
+    want = h + ops.linear_native(x, w, kernel=2)
+    ops.linear_native(x, w, out=h, accum=True, kernel=2)
+    assert torch.equal(h, want), f"{(h != want).sum().item()} of {h.numel()} outputs differ"
