@@ -110,6 +110,20 @@ int rlq_linear_affine_kernel(int kernel, const void *x, int x_stride, int M, int
                              float *y, int y_stride, int accum,
                              void *workspace, size_t workspace_bytes, void *stream);
 
+/* The prefill GEMM is three kernels that give a row the same bits: FULL (128 x 256 output
+ * tiles), MID32 and MID64 (32 or 64 rows x 128, calls with too few of those tiles) and FEW
+ * (32 x 32, affine weights, a few rows). rlq_prefill_route returns the one a call of these
+ * sizes runs (book 0 for affine weights; for a weight whose K is split, of its first rows;
+ * 0 for sizes no call takes). The _prefill entry points run the one named, for tests and
+ * measurement, with the contract of rlq_linear_affine; a kernel that cannot take the call
+ * (FEW for native weights; too few counters for a split weight's tiles) is an error. */
+enum { RLQ_PREFILL_AUTO = 0, RLQ_PREFILL_FULL = 1, RLQ_PREFILL_MID32 = 2, RLQ_PREFILL_MID64 = 3, RLQ_PREFILL_FEW = 4 };
+int rlq_prefill_route(int book, int M, int K, int N);
+int rlq_linear_affine_prefill(int route, const void *x, int x_stride, int M, int K, int N,
+                              const void *packed, int scale_dtype,
+                              float *y, int y_stride, int accum,
+                              void *workspace, size_t workspace_bytes, void *stream);
+
 /* ---------------------------------------------------------------- native 4-bit linear */
 
 /* The native ("q4n") format: a 4-bit codebook value per weight, one fp32 scale per output
@@ -138,6 +152,9 @@ int rlq_linear_native(const void *x, int x_stride, int M, int K, int N, const vo
 int rlq_linear_native_kernel(int kernel, const void *x, int x_stride, int M, int K, int N, const void *packed,
                              const float *s_row, int book, float *y, int y_stride, int accum, void *workspace,
                              size_t workspace_bytes, void *stream);
+int rlq_linear_native_prefill(int route, const void *x, int x_stride, int M, int K, int N, const void *packed,
+                              const float *s_row, int book, float *y, int y_stride, int accum, void *workspace,
+                              size_t workspace_bytes, void *stream);
 
 /* y[m][n] = sum_k x[m][k] * L[q[n][k]]: the native product without the row scale (or any
  * other epilogue), as linear_q4n_raw computes it to measure what linear_q4n's epilogue costs

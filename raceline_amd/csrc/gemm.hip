@@ -744,9 +744,20 @@ static int launch_gemm4_inst(int accum, dim3 grid, size_t lds, hipStream_t st, c
   return 0;
 }
 
-int run_gemm4(int book, const _Float16 *x, int x_stride, int M, int K, int N, const void *codes, const void *sbq,
-              int sd, const float *srow, float *y, int y_stride, int accum, int *cnt, void *ws, size_t ws_bytes,
-              hipStream_t st) {
+static int mid_route(int book, int M, int K, int N, int S) {
+  const int mt = gemm_mid_tiles(book, M, K, N, S);
+  return mt == 1 ? kRouteMid32 : mt == 2 ? kRouteMid64 : kRouteFull;
+}
+
+int prefill_route(int book, int M, int K, int N) {
+  const int S = gemm_split_of(K, N);
+  if (book == kAffine && gemm_few_fits(M, N, S)) return kRouteFew;
+  return mid_route(book, S > 1 ? std::min(M, split_chunk_rows(N)) : M, K, N, S);
+}
+
+int run_gemm4(int route, int book, const _Float16 *x, int x_stride, int M, int K, int N, const void *codes,
+              const void *sbq, int sd, const float *srow, float *y, int y_stride, int accum, int *cnt, void *ws,
+              size_t ws_bytes, hipStream_t st) {
   const int G = K / kGroup;
   const size_t need = gemm4_workspace(book, M, K, N);
   RLQ_REQUIRE(ws_bytes >= need, "workspace of %zu bytes is smaller than the %zu this call needs", ws_bytes, need);
@@ -760,7 +771,16 @@ int run_gemm4(int book, const _Float16 *x, int x_stride, int M, int K, int N, co
   a.M = M; a.K = K; a.N = N; a.y_stride = y_stride;
   const int S = gemm_split_of(K, N);
   RLQ_REQUIRE(S == 1 || cnt, "prefill kernel: this weight splits K in %d, which needs the workspace's counters", S);
-  const bool few = book == kAffine && gemm_few_fits(M, N, S);
+  // a split weight launches in chunks of rows whose tiles have counters; the rows are
+  // independent, so chunking changes no result
+  const int chunk = S > 1 ? split_chunk_rows(N) : M;
+  RLQ_REQUIRE(route >= kRouteAuto && route <= kRouteFew, "prefill kernel: unknown route %d", route);
+  RLQ_REQUIRE(route != kRouteFew || (book == kAffine && M <= chunk && gemm_few_counters_fit(M, N, S)),
+              "prefill kernel: route %d does not take book %d, M=%d N=%d split %d", route, book, M, N, S);
+  RLQ_REQUIRE((route != kRouteMid32 && route != kRouteMid64) ||
+                  gemm_mid_counters_fit(route == kRouteMid32 ? 1 : 2, std::min(M, chunk), N, S),
+              "prefill kernel: route %d does not take M=%d N=%d split %d", route, M, N, S);
+  const bool few = route == kRouteAuto ? book == kAffine && gemm_few_fits(M, N, S) : route == kRouteFew;
   if (book == kAffine) {
     const int gs_stride = gs_stride_of(G, sd);
     _Float16 *xp = static_cast<_Float16 *>(ws);
@@ -796,9 +816,6 @@ int run_gemm4(int book, const _Float16 *x, int x_stride, int M, int K, int N, co
   if (S > 1) a.y_part = reinterpret_cast<float *>(static_cast<char *>(ws) + books_workspace(book, M, K));
   const int nblocks = (N + kGN - 1) / kGN;
   const size_t lds = (size_t)kGemmLdsBytes;
-  // a split weight launches in chunks of rows whose tiles have counters; the rows are
-  // independent, so chunking changes no result
-  const int chunk = S > 1 ? split_chunk_rows(N) : M;
   for (int r0 = 0; r0 < M; r0 += chunk) {
     GemmArgs c = a;
     c.M = std::min(chunk, M - r0);
@@ -811,8 +828,9 @@ int run_gemm4(int book, const _Float16 *x, int x_stride, int M, int K, int N, co
       if (int rc = launch_gemm_few(sd, c, S, accum, st)) return rc;
       continue;
     }
-    if (const int mt = gemm_mid_tiles(book, c.M, K, N, S)) {   // too few of this kernel's tiles to fill the chip
-      if (int rc = launch_gemm_mid(book, sd, mt, c, S, accum, st)) return rc;
+    const int r = route == kRouteAuto ? mid_route(book, c.M, K, N, S) : route;
+    if (r != kRouteFull) {   // too few of this kernel's tiles to fill the chip
+      if (int rc = launch_gemm_mid(book, sd, r == kRouteMid32 ? 1 : 2, c, S, accum, st)) return rc;
       continue;
     }
     const dim3 grid((c.M + kGM - 1) / kGM * nblocks, S);

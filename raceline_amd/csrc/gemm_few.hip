@@ -316,6 +316,7 @@ static long long few_tiles(int M, int N, int S, int rb) {
   return (long long)((N + 31) / 32) * ((M + rb - 1) / rb) * S;
 }
 bool gemm_few_fits(int M, int N, int S) { return few_tiles(M, N, S, 32) <= kFewMaxTiles; }
+bool gemm_few_counters_fit(int M, int N, int S) { return S == 1 || few_tiles(M, N, 1, 32) <= kGemmMaxCounters; }
 
 int launch_gemm_few(int sd, const GemmArgs &a, int S, int accum, hipStream_t st) {
   static LdsOptIn o0, o1;

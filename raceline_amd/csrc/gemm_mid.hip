@@ -437,6 +437,11 @@ constexpr MidCost kCostAffine[3] = {{5.7, 1.48, 0.38}, {10.5, 0.25, 0.10}, {13.5
 constexpr MidCost kCostInt[3] = {{3.4, 1.33, 0.41}, {7.4, 0.35, 0.0}, {6.5, 0.43, 0.07}};
 constexpr MidCost kCostFp4[3] = {{8.0, 1.5, 0.7}, {6.0, 0.40, 0.0}, {6.0, 0.63, 0.0}};
 
+// a split call's tiles count their arrivals in the workspace's counters
+bool gemm_mid_counters_fit(int mt, int M, int N, int S) {
+  return S == 1 || (long long)((M + 32 * mt - 1) / (32 * mt)) * ((N + kMidCols - 1) / kMidCols) <= kGemmMaxCounters;
+}
+
 int gemm_mid_tiles(int book, int M, int K, int N, int S) {
   const MidCost *cost = book == kAffine ? kCostAffine : book == kFp4 ? kCostFp4 : kCostInt;
   const double pairs = ((K / kGroup + 1) / 2 + S - 1) / S;
@@ -447,10 +452,8 @@ int gemm_mid_tiles(int book, int M, int K, int N, int S) {
   const double t4 = time(cost[0], (long long)((N + 255) / 256) * ((M + 127) / 128) * S, 256);
   const double t1 = time(cost[1], nt * ((M + 31) / 32) * S, 1024);
   const double t2 = time(cost[2], nt * ((M + 63) / 64) * S, 1024);
-  // a split call's tiles count their arrivals in the workspace's counters
-  auto fits = [&](int mt) { return S == 1 || (long long)((M + 32 * mt - 1) / (32 * mt)) * ((N + kMidCols - 1) / kMidCols) <= kGemmMaxCounters; };
-  if (t1 <= t2 && t1 < t4 && fits(1)) return 1;
-  return t2 < t4 && fits(2) ? 2 : 0;
+  if (t1 <= t2 && t1 < t4 && gemm_mid_counters_fit(1, M, N, S)) return 1;
+  return t2 < t4 && gemm_mid_counters_fit(2, M, N, S) ? 2 : 0;
 }
 
 int launch_gemm_mid(int book, int sd, int mt, const GemmArgs &a, int S, int accum, hipStream_t st) {

@@ -15,7 +15,7 @@ inline size_t packed_tile_sb_offset(int K, int t) { return (size_t)t * quads_of(
 
 // y (+)= x W^T for the packed matrix (or row range) whose sections start at codes and sbq
 // (sbq unused for native books, whose row scales are srow). kernel: 0 automatic, 1 decode,
-// 2 prefill; book: kAffine or a native codebook; sd: RLQ_F16 / RLQ_BF16. Arguments are
+// 2 prefill (2 + a PrefillRoute of gemm.h: that prefill kernel); book: kAffine or a native codebook; sd: RLQ_F16 / RLQ_BF16. Arguments are
 // the caller's to check (the entry points of linear.hip do).
 int linear_packed(int kernel, int book, const _Float16 *x, int x_stride, int M, int K, int N, const void *codes,
                   const void *sbq, int sd, const float *srow, float *y, int y_stride, int accum, void *ws,

@@ -767,7 +767,7 @@ int linear_swiglu_packed(const _Float16 *x, int x_stride, int M, int K, int I, c
 int linear_packed(int kernel, int book, const _Float16 *x, int x_stride, int M, int K, int N, const void *codes,
                   const void *sbq, int sd, const float *srow, float *y, int y_stride, int accum, void *ws,
                   size_t ws_bytes, hipStream_t st) {
-  RLQ_REQUIRE(kernel >= 0 && kernel <= 2, "unknown kernel %d", kernel);
+  RLQ_REQUIRE(kernel >= 0 && kernel <= 2 + kRouteFew, "unknown kernel %d", kernel);
   // the workspace: split counters first, then the decode partials or the prefill kernel's data
   const bool has_ws = ws && ws_bytes >= kGemvCountBytes;
   int *cnt = has_ws ? static_cast<int *>(ws) : nullptr;
@@ -777,7 +777,7 @@ int linear_packed(int kernel, int book, const _Float16 *x, int x_stride, int M, 
   if (gemv)
     return run_gemv(book, x, x_stride, M, K, N, codes, sbq, sd, srow, y, y_stride, accum, cnt,
                     static_cast<float *>(rest), rest_bytes, st);
-  return run_gemm4(book, x, x_stride, M, K, N, codes, sbq, sd, srow, y, y_stride, accum, cnt, rest, rest_bytes, st);
+  return run_gemm4(std::max(kernel - 2, 0), book, x, x_stride, M, K, N, codes, sbq, sd, srow, y, y_stride, accum, cnt, rest, rest_bytes, st);
 }
 
 // ================================================================== group sums
@@ -944,18 +944,34 @@ int rlq_pack_native_blocked(const uint8_t *w_blk, int K, int n_pad, int row0, in
   return 0;
 }
 
-int rlq_linear_native_kernel(int kernel, const void *x, int x_stride, int M, int K, int N, const void *packed,
-                             const float *s_row, int book, float *y, int y_stride, int accum, void *workspace,
-                             size_t workspace_bytes, void *stream) {
+// kernel: as for linear_packed, checked by the entry points below
+static int linear_native(int kernel, const void *x, int x_stride, int M, int K, int N, const void *packed,
+                         const float *s_row, int book, float *y, int y_stride, int accum, void *workspace,
+                         size_t workspace_bytes, void *stream) {
   int rc = check_linear_args("rlq_linear_native", x, x_stride, M, K, N, packed, RLQ_F16, y, y_stride);
   if (rc) return rc;
   RLQ_REQUIRE(book == RLQ_BOOK_INT15 || book == RLQ_BOOK_INT16 || book == RLQ_BOOK_FP4,
               "rlq_linear_native: unknown codebook %d", book);
   RLQ_REQUIRE(s_row && aligned(s_row, 4), "rlq_linear_native: null or misaligned row scales");
-  RLQ_REQUIRE(kernel >= 0 && kernel <= 2, "rlq_linear_native_kernel: unknown kernel %d", kernel);
   // native matrices have no scale/bias section: the codes stand in for it (never read)
   return linear_packed(kernel, book, static_cast<const _Float16 *>(x), x_stride, M, K, N, packed, packed, RLQ_F16,
                        s_row, y, y_stride, accum, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+int rlq_linear_native_kernel(int kernel, const void *x, int x_stride, int M, int K, int N, const void *packed,
+                             const float *s_row, int book, float *y, int y_stride, int accum, void *workspace,
+                             size_t workspace_bytes, void *stream) {
+  RLQ_REQUIRE(kernel >= 0 && kernel <= 2, "rlq_linear_native_kernel: unknown kernel %d", kernel);
+  return linear_native(kernel, x, x_stride, M, K, N, packed, s_row, book, y, y_stride, accum, workspace,
+                       workspace_bytes, stream);
+}
+
+int rlq_linear_native_prefill(int route, const void *x, int x_stride, int M, int K, int N, const void *packed,
+                              const float *s_row, int book, float *y, int y_stride, int accum, void *workspace,
+                              size_t workspace_bytes, void *stream) {
+  RLQ_REQUIRE(route >= kRouteAuto && route <= kRouteFew, "rlq_linear_native_prefill: unknown route %d", route);
+  return linear_native(2 + route, x, x_stride, M, K, N, packed, s_row, book, y, y_stride, accum, workspace,
+                       workspace_bytes, stream);
 }
 
 int rlq_linear_native_raw(const void *x, int x_stride, int M, int K, int N, const void *packed, int book, float *y,
@@ -983,15 +999,35 @@ size_t rlq_linear_workspace_bytes(int M, int K, int N) {
                                      gemm4_workspace(kInt16, M, K, N), gemm4_workspace(kInt15, M, K, N)});
 }
 
-int rlq_linear_affine_kernel(int kernel, const void *x, int x_stride, int M, int K, int N, const void *packed,
-                             int scale_dtype, float *y, int y_stride, int accum, void *workspace,
-                             size_t workspace_bytes, void *stream) {
+int rlq_prefill_route(int book, int M, int K, int N) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % kGroup || book < kAffine || book > kFp4) return 0;
+  return prefill_route(book, M, K, N);
+}
+
+static int linear_affine(int kernel, const void *x, int x_stride, int M, int K, int N, const void *packed,
+                         int scale_dtype, float *y, int y_stride, int accum, void *workspace, size_t workspace_bytes,
+                         void *stream) {
   int rc = check_linear_args("rlq_linear_affine", x, x_stride, M, K, N, packed, scale_dtype, y, y_stride);
   if (rc) return rc;
-  RLQ_REQUIRE(kernel >= 0 && kernel <= 2, "rlq_linear_affine_kernel: unknown kernel %d", kernel);
   const void *sbq = static_cast<const char *>(packed) + packed_code_bytes(K, N);
   return linear_packed(kernel, kAffine, static_cast<const _Float16 *>(x), x_stride, M, K, N, packed, sbq, scale_dtype,
                        nullptr, y, y_stride, accum, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+int rlq_linear_affine_kernel(int kernel, const void *x, int x_stride, int M, int K, int N, const void *packed,
+                             int scale_dtype, float *y, int y_stride, int accum, void *workspace,
+                             size_t workspace_bytes, void *stream) {
+  RLQ_REQUIRE(kernel >= 0 && kernel <= 2, "rlq_linear_affine_kernel: unknown kernel %d", kernel);
+  return linear_affine(kernel, x, x_stride, M, K, N, packed, scale_dtype, y, y_stride, accum, workspace,
+                       workspace_bytes, stream);
+}
+
+int rlq_linear_affine_prefill(int route, const void *x, int x_stride, int M, int K, int N, const void *packed,
+                              int scale_dtype, float *y, int y_stride, int accum, void *workspace,
+                              size_t workspace_bytes, void *stream) {
+  RLQ_REQUIRE(route >= kRouteAuto && route <= kRouteFew, "rlq_linear_affine_prefill: unknown route %d", route);
+  return linear_affine(2 + route, x, x_stride, M, K, N, packed, scale_dtype, y, y_stride, accum, workspace,
+                       workspace_bytes, stream);
 }
 
 int rlq_linear_affine(const void *x, int x_stride, int M, int K, int N, const void *packed, int scale_dtype, float *y,

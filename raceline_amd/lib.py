@@ -35,6 +35,11 @@ SIGNATURES = {
                                   c_void_p, c_size_t, c_void_p]),
     "rlq_linear_affine_kernel": (c_int, [c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p,
                                          c_int, c_int, c_void_p, c_size_t, c_void_p]),
+    "rlq_prefill_route": (c_int, [c_int, c_int, c_int, c_int]),
+    "rlq_linear_affine_prefill": (c_int, [c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p,
+                                          c_int, c_int, c_void_p, c_size_t, c_void_p]),
+    "rlq_linear_native_prefill": (c_int, [c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int,
+                                          c_void_p, c_int, c_int, c_void_p, c_size_t, c_void_p]),
     "rlq_group_sums": (c_int, [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p]),
     "rlq_dequant_affine": (c_int, [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p]),
     "rlq_stream_read": (c_int, [c_void_p, c_size_t, c_void_p, c_void_p]),
@@ -113,7 +118,7 @@ def library_path() -> str:
                        "(or __graft_entry__.build()) or point RACELINE_LIB at it")
 
 
-_STATUS_FREE = ("rlq_abi_version", "rlq_set_fatal")   # int results that are no status
+_STATUS_FREE = ("rlq_abi_version", "rlq_set_fatal", "rlq_prefill_route")   # int results that are no status
 
 
 @functools.lru_cache(maxsize=1)

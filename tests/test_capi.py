@@ -123,6 +123,27 @@ def test_raw_native_product_refuses_the_half_step_book():
         lib.call("rlq_linear_native_raw", 16, 64, 1, 64, 16, 16, 2, 16, 16, None, 0, None)
 
 
+def test_prefill_kernel_that_cannot_take_the_call_is_refused():
+    """Naming a prefill kernel that cannot take the call is an error before any launch (pointers
+    are placeholders, never dereferenced): the few-row kernel for native weights, a split weight
+    with more tiles than counters (K = 8192, N = 5120 splits in two), an unknown one."""
+    big = 1 << 32
+    native = (16, 64, 32, 64, 64, 16, 16, 1, 16, 64, 0, 256, big, None)
+    with pytest.raises(lib.RlqError, match="does not take"):
+        lib.call("rlq_linear_native_prefill", 4, *native)
+    split = (16, 8192, 1100, 8192, 5120, 16, 0, 16, 5120, 0, 256, big, None)
+    for route in (2, 4):
+        with pytest.raises(lib.RlqError, match="does not take"):
+            lib.call("rlq_linear_affine_prefill", route, *split)
+    for route in (-1, 5):
+        with pytest.raises(lib.RlqError, match="unknown route"):
+            lib.call("rlq_linear_affine_prefill", route, *split)
+        with pytest.raises(lib.RlqError, match="unknown route"):
+            lib.call("rlq_linear_native_prefill", route, *native)
+    assert lib.call("rlq_prefill_route", 0, 64, 100, 64) == 0
+    assert lib.call("rlq_prefill_route", 4, 64, 128, 64) == 0
+
+
 def test_calls_follow_a_reloaded_library(tmp_path, monkeypatch):
     """After load.cache_clear() (a library rebuilt in the same process) calls, their error mode
     and their messages all come from the library that load() then gives, not from the one the
