@@ -43,6 +43,7 @@ constexpr int kFewPairBytes = 2 * 4 * 1024;           // a pair's products: [gro
 constexpr int kFewScaleBytes = 512;                   // and its scale words: [lane] 8 bytes
 constexpr int kFewSetBytes = kFewProducers * (kFewPairBytes + kFewScaleBytes);
 constexpr int kFewMaxTiles = 256;                     // a workgroup per CU
+constexpr int kFewMaxRows = 2048;
 constexpr int kFewLds = 2 * kFewSetBytes;             // 136 KB: one workgroup per CU
 
 // What a producer wave reads (see few_codes, few_frag).
@@ -311,11 +312,14 @@ __global__ __launch_bounds__(kFewThreads, 3) void gemm_few_kernel(GemmArgs a, in
 // Taken where the call's tiles fill the CUs once at most (a workgroup is a CU's worth of waves
 // and LDS): a second round costs a whole workgroup's time again, which the streaming kernels
 // do not pay (4096 x 4096 at 96 rows, 384 tiles: 23.5 us against gemm_mid_kernel's 20.3; at
-// 64 rows, 256 tiles: 14.8 against 20.1).
+// 64 rows, 256 tiles: 14.8 against 20.1). Tall, narrow calls stay with those too: the prep
+// pass writes each row's chunks 16 M bytes apart, eight rows to a cache line, which costs more
+// than the GEMM gains past about 2000 rows (f16 K = 2752 .. 13504, N = 21 .. 39: 3043 rows 35.1
+// us against 29.0, 3905 135.8 against 61.2, 8191 60.2 against 33.0; 1929 rows 27.1 against 28.0).
 static long long few_tiles(int M, int N, int S, int rb) {
   return (long long)((N + 31) / 32) * ((M + rb - 1) / rb) * S;
 }
-bool gemm_few_fits(int M, int N, int S) { return few_tiles(M, N, S, 32) <= kFewMaxTiles; }
+bool gemm_few_fits(int M, int N, int S) { return M <= kFewMaxRows && few_tiles(M, N, S, 32) <= kFewMaxTiles; }
 bool gemm_few_counters_fit(int M, int N, int S) { return S == 1 || few_tiles(M, N, 1, 32) <= kGemmMaxCounters; }
 
 int launch_gemm_few(int sd, const GemmArgs &a, int S, int accum, hipStream_t st) {

@@ -144,6 +144,16 @@ def test_prefill_kernel_that_cannot_take_the_call_is_refused():
     assert lib.call("rlq_prefill_route", 4, 64, 128, 64) == 0
 
 
+def test_prefill_kernel_of_tall_narrow_calls():
+    """The few-row kernel takes calls of at most 256 tiles of 32 x 32 and 2048 rows: with more
+    rows its prep pass costs more than it gains (3905 x 13504 x 21: 136 us against 61)."""
+    def route(M, K, N):
+        return lib.call("rlq_prefill_route", 0, M, K, N)
+
+    assert all(route(*c) == 4 for c in ((9, 4096, 4096), (64, 4096, 4096), (2048, 4096, 64), (1024, 512, 256)))
+    assert all(route(*c) in (1, 2, 3) for c in ((65, 4096, 4096), (2049, 4096, 32), (3905, 13504, 21), (8192, 4096, 32)))
+
+
 def test_calls_follow_a_reloaded_library(tmp_path, monkeypatch):
     """After load.cache_clear() (a library rebuilt in the same process) calls, their error mode
     and their messages all come from the library that load() then gives, not from the one the
