@@ -22,6 +22,7 @@
 #include "../../include/rlq.h"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 #include <utility>
 
@@ -420,22 +421,38 @@ static int launch_mid_rows(int mt, const GemmArgs &a, int S, int accum, hipStrea
 }
 
 // Which kernel and tile take a call: the one of three estimated fastest (32 or 64 rows x 128
-// features here, gemm4_kernel's 128 x 256), each as
-//   once + group pairs per workgroup x (per_round x rounds of the chip + per_fill x units / units of a round),
-// in us, fitted to launches timed with their prep pass on 9B and 27B projections (K 4096 ..
-// 12288, N 4096 .. 34816) at M = 16 .. 1024. A wave here is bound by its own instruction
-// issue, and two resident on a SIMD take about as long as one after the other, so the rounds
-// count; how full they are costs memory time and clock. The books differ in what a code
-// costs to convert (4 operations for eight fp4 codes, 13 for eight integer ones, shared by two row
-// tiles at 64 rows), the affine one in its scale FMAs. Against the fastest of the three at 65
-// shapes a book, the choice loses 0.3% on average and 4% at most (affine), 0.1% and 4%
-// (integer books), 0.2% and 6% (fp4); one set of constants for all books lost up to 12% and
-// 30%: int15 K = 5120, N = 34816 at M = 48 took the 32-row tile, 49.4 us, for the 64-row
-// tile's 38.1; affine K = 4096, N = 24576 at M = 256 the 64-row tile, 67.8, for gemm4's 60.4.
-struct MidCost { double once, per_round, per_fill; };
-constexpr MidCost kCostAffine[3] = {{5.7, 1.48, 0.38}, {10.5, 0.25, 0.10}, {13.5, 0.41, 0.15}};   // gemm4, 32 rows, 64 rows
-constexpr MidCost kCostInt[3] = {{3.4, 1.33, 0.41}, {7.4, 0.35, 0.0}, {6.5, 0.43, 0.07}};
-constexpr MidCost kCostFp4[3] = {{8.0, 1.5, 0.7}, {6.0, 0.40, 0.0}, {6.0, 0.63, 0.0}};
+// features here, gemm4_kernel's 128 x 256), each as, in us,
+//   once + pairs x (per_round x rounds of the chip + per_fill x fill) + (per_tile + split (S - 1)) x fill
+// with fill = units / units of a round, rounds = fill rounded up, and the group pairs of a
+// workgroup rounded up to the ones its loop runs (3, 8 or 4 LDS stages). A wave here is bound by
+// its own instruction issue, and two resident on a SIMD take about as long as one after the
+// other, so the rounds count; how full they are costs memory time and clock.
+// The tiles here have one more term. Each 128 features read all rows, which an XCD's L2 (4 MB)
+// holds for small calls; rows beyond it come from memory once per 128 features, at row_mb us per
+// MB (from 2 MB of rows on, in full from 12 MB). The native books' waves have little to do
+// beside those loads and pay the sum, the affine ones' scale FMAs hide most of the shorter of
+// the two (the cube root of the sum of cubes). gemm4_kernel orders its tiles in blocks of 512
+// rows and shows no such term.
+// The books differ in what a code costs to convert (4 operations for eight fp4 codes, 13 for
+// eight integer ones, shared by two row tiles at 64 rows), the affine one in its scale FMAs,
+// int16 in the launch that sums its rows first. Fitted to launches timed with their prep pass:
+// K 128 .. 17408 (odd numbers of groups and split weights among them), N 16 .. 34816, 9 .. 4096
+// rows (to 16384 where N < 256), 828 calls (affine), 431 (int15), 467 (int16) and 470 (fp4).
+// Against the fastest of the three the choice loses 0.3%, 0.1%, 0.3% and 0.4% on average and at
+// most 11%, 16%, 20% and 19%; against gemm4_kernel before it shared the work (as slow for large
+// calls and 5% slower) 1.4% at one call and nothing at the rest. Without the rows' term, the
+// rounding of the pairs and the split it took the 64-row tiles for large calls: bf16 K = 16512,
+// N = 2187 at 2762 rows 383 us for gemm4's 266, fp4 K = 2240, N = 3877 at 1600 rows 46.1 for 36.5.
+struct MidCost { double once, per_round, per_fill, per_tile, split, row_mb; };
+constexpr MidCost kCost[4][3] = {   // by book; gemm4, 32 rows, 64 rows
+    {{9.2, 1.386, 0.49, 5.4, 15.8, 0.0}, {10.0, 0.366, 0.0, 0.5, 1.6, 0.1173}, {14.5, 0.413, 0.151, 1.6, 2.4, 0.1145}},
+    {{4.0, 1.214, 0.339, 7.6, 9.5, 0.0}, {5.0, 0.349, 0.0, 0.4, 0.6, 0.0057}, {4.5, 0.478, 0.0, 1.6, 2.0, 0.0118}},
+    {{10.5, 1.253, 0.557, 4.5, 15.7, 0.0}, {8.3, 0.356, 0.0, 0.3, 2.9, 0.013}, {7.9, 0.489, 0.0, 1.4, 3.7, 0.0158}},
+    {{4.6, 1.03, 0.421, 7.5, 8.2, 0.0}, {4.1, 0.212, 0.016, 1.1, 0.0, 0.0238}, {4.2, 0.336, 0.016, 2.4, 0.2, 0.0248}}};
+static_assert(kAffine == 0 && kInt15 == 1 && kInt16 == 2 && kFp4 == 3, "kCost's rows");
+// what gemm4_kernel may be slower by and still take a call: estimates closer than this pick
+// either, and its times vary less
+constexpr double kMidMargin = 1.02;
 
 // a split call's tiles count their arrivals in the workspace's counters
 bool gemm_mid_counters_fit(int mt, int M, int N, int S) {
@@ -443,15 +460,21 @@ bool gemm_mid_counters_fit(int mt, int M, int N, int S) {
 }
 
 int gemm_mid_tiles(int book, int M, int K, int N, int S) {
-  const MidCost *cost = book == kAffine ? kCostAffine : book == kFp4 ? kCostFp4 : kCostInt;
-  const double pairs = ((K / kGroup + 1) / 2 + S - 1) / S;
-  auto time = [&](const MidCost &c, long long units, int per) {
-    return c.once + pairs * (c.per_round * (double)((units + per - 1) / per) + c.per_fill * (double)units / per);
+  const int pairs = ((K / kGroup + 1) / 2 + S - 1) / S;
+  const double rows_mb = 2e-6 * M * K, beyond = std::clamp((rows_mb - 2.0) / 10.0, 0.0, 1.0);
+  const double read = rows_mb * ((N + kMidCols - 1) / kMidCols) * beyond;
+  auto time = [&](const MidCost &c, long long units, int per, int stages) {
+    const double fill = (double)units / per, rounds = (double)((units + per - 1) / per);
+    const double run = (double)((pairs + stages - 1) / stages * stages);
+    const double work = run * (c.per_round * rounds + c.per_fill * fill) + (c.per_tile + c.split * (S - 1)) * fill;
+    const double rows = c.row_mb * read;
+    return c.once + (book == kAffine ? std::cbrt(work * work * work + rows * rows * rows) : work + rows);
   };
+  const MidCost *cost = kCost[book];
   const long long nt = (N + 31) / 32;
-  const double t4 = time(cost[0], (long long)((N + 255) / 256) * ((M + 127) / 128) * S, 256);
-  const double t1 = time(cost[1], nt * ((M + 31) / 32) * S, 1024);
-  const double t2 = time(cost[2], nt * ((M + 63) / 64) * S, 1024);
+  const double t4 = time(cost[0], (long long)((N + 255) / 256) * ((M + 127) / 128) * S, 256, 3);
+  const double t1 = kMidMargin * time(cost[1], nt * ((M + 31) / 32) * S, 1024, mid_ring<1>());
+  const double t2 = kMidMargin * time(cost[2], nt * ((M + 63) / 64) * S, 1024, mid_ring<2>());
   if (t1 <= t2 && t1 < t4 && gemm_mid_counters_fit(1, M, N, S)) return 1;
   return t2 < t4 && gemm_mid_counters_fit(2, M, N, S) ? 2 : 0;
 }
