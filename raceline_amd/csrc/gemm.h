@@ -30,6 +30,10 @@ constexpr int kGemmMaxCounters = 1024;
 // sums; kInt16: row sums; a shape whose K is split: the partial products).
 size_t gemm4_workspace(int book, int M, int K, int N);
 
+// Affine: steps of the bias product that run before the K loop, the rest after it. A row's bits
+// depend on the number, so all prefill kernels share it (it is what fits gemm4_kernel's stage 2).
+constexpr int kBiasProSteps = 11;
+
 // The prefill kernels and their tiles, with the same bits for every row; kRouteAuto takes the
 // one estimated fastest (run_gemm4, gemm_mid_tiles).
 enum PrefillRoute { kRouteAuto = 0, kRouteFull = 1, kRouteMid32 = 2, kRouteMid64 = 3, kRouteFew = 4 };

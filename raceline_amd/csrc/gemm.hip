@@ -48,8 +48,7 @@ constexpr int kStages = 3;                  // loads run two group pairs ahead o
 constexpr int kGroupM = 4;                  // token blocks per group of the workgroup order
 constexpr int kBiasChunk = 32;              // bias product: steps of group-sum pieces staged at a time
 constexpr int kMaxGemmSplit = 2;            // workgroups per output tile when K is split
-constexpr int kProBiasSteps = 11;           // bias steps run in the prologue (their pieces fill 47 KB)
-static_assert(kGM * (32 * kProBiasSteps + 16) <= kABytes + kBBytes, "the prologue's bias pieces fit stage 2");
+static_assert(kGM * (32 * kBiasProSteps + 16) <= kABytes + kBBytes, "the prologue's bias pieces (47 KB) fit stage 2");
 // LDS by part, then stage: the three activation tiles, the three code parts, the three
 // scale parts, so that with the stage known at compile time every read of a stage is a
 // lane's base address plus an immediate offset
@@ -434,14 +433,14 @@ __global__ __launch_bounds__(kGThreads) void gemm4_kernel(GemmArgs a) {
   // per workgroup, cs steps at a time, rows padded by 16 bytes (an odd number of 16-byte
   // slots apart, so the fragment reads of 32 rows spread over the banks). Each wave's scale
   // quads (its own biases) come straight from memory, in flight while the pieces land.
-  // The first kProBiasSteps steps run in the prologue, their loads in flight with the first
+  // The first kBiasProSteps steps run in the prologue, their loads in flight with the first
   // two stages' (one wait for both), the pieces in stage 2's activation and code parts, free
   // until stage 2 is issued: as the workgroup's last phase the bias product cost the whole
   // round trip of its loads (27B gate_up at M = 2048: 116 us of 865). Later steps (long K,
   // bf16 biases) run at the end, from the start of the LDS.
   const int bsteps = a.gs_stride / 16;
   const int st_lo = split * bsteps / S, st_hi = (split + 1) * bsteps / S;
-  const int st_pro = BOOK == kAffine ? min(st_hi, st_lo + kProBiasSteps) : st_lo;
+  const int st_pro = BOOK == kAffine ? min(st_hi, st_lo + kBiasProSteps) : st_lo;
   auto bias_chunk = [&](int st0, int cs, bool pro) {
     const int tn = t0 + 2 * wave;
     const int tv = max(0, min(T, tn + 2) - tn);

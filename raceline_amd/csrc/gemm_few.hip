@@ -37,7 +37,6 @@ namespace rlq {
 
 constexpr int kFewProducers = 8, kFewAccs = 4;
 constexpr int kFewThreads = 64 * (kFewProducers + kFewAccs);
-constexpr int kFewBiasPro = 11;                       // bias steps before the K loop, as gemm4_kernel runs them
 constexpr int kFewBiasChunk = 8;
 constexpr int kFewPairBytes = 2 * 4 * 1024;           // a pair's products: [group][quarter of the rows][lane] 16 bytes
 constexpr int kFewScaleBytes = 512;                   // and its scale words: [lane] 8 bytes
@@ -192,7 +191,7 @@ __global__ __launch_bounds__(kFewThreads, 3) void gemm_few_kernel(GemmArgs a, in
   const int quarter = wave - kFewProducers;               // accumulator wave: rows 8 quarter .. + 7 of the tile
   const int bsteps = a.gs_stride / 16;
   const int st_lo = split * bsteps / S, st_hi = (split + 1) * bsteps / S;
-  const int st_pro = min(st_hi, st_lo + kFewBiasPro);
+  const int st_pro = min(st_hi, st_lo + kBiasProSteps);
   const int n = 32 * nb + c32, nc = min(n, a.N - 1);
   const bool col = n < a.N;
   const int mrow = m0 + 8 * quarter + 4 * h;              // the lane's first row; registers 4 quarter + 0 .. 3 of the tile
@@ -206,7 +205,7 @@ __global__ __launch_bounds__(kFewThreads, 3) void gemm_few_kernel(GemmArgs a, in
     const bool rows = quarter < quarters;                 // uniform: the wave has rows to sum
     f32x16 full[1] = {f32x16{}};
     if (rows) {
-      u32x4 bv[kFewBiasPro], ba[kFewBiasPro][1];
+      u32x4 bv[kBiasProSteps], ba[kBiasProSteps][1];
       bias_load<SD, 1>(bias, bv, ba, st_lo, st_pro);
       bias_mul<SD, 1>(bv, ba, h, full);
     }

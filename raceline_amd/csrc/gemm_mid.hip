@@ -31,7 +31,6 @@ namespace rlq {
 constexpr int kMidWaves = 4;             // (two per workgroup measured the same on small grids, up to 1.6 times slower on full ones)
 constexpr int kMidCols = 32 * kMidWaves; // features of a workgroup
 constexpr int kMidRow = 256;             // LDS bytes of one row of a stage: one pair of groups, 128 fp16
-constexpr int kMidBiasPro = 11;          // bias steps before the K loop, as gemm4_kernel runs them
 constexpr int kMidBiasChunk = 8;         // bias steps loaded at a time after it
 
 template <int MT> constexpr int mid_stage_bytes() { return 32 * MT * kMidRow; }
@@ -153,7 +152,7 @@ __global__ __launch_bounds__(64 * kMidWaves, 2) void gemm_mid_kernel(GemmArgs a,
   // the range load zeros and add nothing.
   const int bsteps = a.gs_stride / 16;
   const int st_lo = split * bsteps / S, st_hi = (split + 1) * bsteps / S;
-  const int st_pro = BOOK == kAffine ? min(st_hi, st_lo + kMidBiasPro) : st_lo;
+  const int st_pro = BOOK == kAffine ? min(st_hi, st_lo + kBiasProSteps) : st_lo;
   BiasSrc bias;
   bias.rgs = make_rsrc(a.gs, BOOK == kAffine ? (uint32_t)((size_t)a.M * a.gs_stride * 2) : 0u);
   bias.rsb = make_rsrc(src.s, src.srange);
@@ -173,7 +172,7 @@ __global__ __launch_bounds__(64 * kMidWaves, 2) void gemm_mid_kernel(GemmArgs a,
     }
   };
   if constexpr (BOOK == kAffine) {
-    u32x4 bv[kMidBiasPro], ba[kMidBiasPro][MT];
+    u32x4 bv[kBiasProSteps], ba[kBiasProSteps][MT];
     bias_load<SD, MT>(bias, bv, ba, st_lo, st_pro);
     __builtin_amdgcn_sched_barrier(0);        // requested before the ring: they complete first
     fill();

@@ -807,10 +807,12 @@ __global__ void group_sums_kernel(const _Float16 *x, int x_stride, int M, int K,
 
 // asum[m] = the sum over a row's groups, in order, of their sums (each summed in order too):
 // the activation row sums the half-step codebook needs. One workgroup per row: a thread sums
-// a group, one thread adds the group sums from the LDS. Bound by its launch and that chain
-// of adds (latency): with a launch for the group sums and one thread per row adding them from
-// memory, int16 calls of 16 rows
-// took 18 us longer than int15 ones at K = 4096 and 47 at K = 12288, now 3.
+// a group, one thread adds the group sums from the LDS. Bound at few rows by its launch and
+// that chain of adds (latency): with a launch for the group sums and one thread per row adding
+// them from memory, int16 calls of 16 rows took 19 us longer than int15 ones at K = 4096 and 47
+// at K = 12288, now 3 and 4. At many rows by its loads: a thread reads its group's 128 bytes, so
+// a wave's loads lie 128 bytes apart; 2048 rows cost 7 to 12 us at K = 4096 (38 before) and 50
+// to 56 at K = 12288 (116 before).
 constexpr int kRowSumChunk = 1024;   // group sums in the LDS at a time
 __global__ void row_sums_kernel(const _Float16 *x, int x_stride, int K, float *asum) {
   __shared__ f32x4 gs[kRowSumChunk / 4];
