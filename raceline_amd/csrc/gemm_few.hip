@@ -20,7 +20,7 @@
 // runs of rows and a wave needs no LDS stage to transpose through. Rows past M load as
 // zeros; products of rows that do not exist are not written to the LDS (8 rows at a time).
 //
-// What bounds it: the CU's vector memory path (TA 77%, TD 88% busy at K = 12288, 32 rows), of
+// What bounds it: the CU's vector memory path (TA 77%, TD 89% busy at K = 12288, 27 rows), of
 // which the activations are four fifths (8 KB a pair, the codes 2.3 KB). So where the chip has
 // CUs to spare a workgroup takes 16 or 8 rows and others the rest. Measured with the prep pass,
 // against gemm_mid_kernel: 4096 x 4096 at 9 / 32 / 64 rows 11.5 / 12.4 / 14.8 us (18.7, 19.4,
