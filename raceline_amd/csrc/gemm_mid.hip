@@ -438,10 +438,11 @@ static int launch_mid_rows(int mt, const GemmArgs &a, int S, int accum, hipStrea
 // K 128 .. 17408 (odd numbers of groups and split weights among them), N 16 .. 34816, 9 .. 4096
 // rows (to 16384 where N < 256), 828 calls (affine), 431 (int15), 467 (int16) and 470 (fp4).
 // Against the fastest of the three the choice loses 0.3%, 0.1%, 0.3% and 0.4% on average and at
-// most 11%, 16%, 20% and 19%; against gemm4_kernel before it shared the work (as slow for large
-// calls and 5% slower) 1.4% at one call and nothing at the rest. Without the rows' term, the
-// rounding of the pairs and the split it took the 64-row tiles for large calls: bf16 K = 16512,
-// N = 2187 at 2762 rows 383 us for gemm4's 266, fp4 K = 2240, N = 3877 at 1600 rows 46.1 for 36.5.
+// most 11%, 16%, 20% and 19%. Of these calls and 1423 others drawn afterwards three are slower
+// than on gemm4_kernel alone as it was before the tiles here (1.4%, 1.5% and 3.1%). Without the
+// rows' term, the rounding of the pairs and the split it took the 64-row tiles for large calls:
+// bf16 K = 16512, N = 2187 at 2762 rows 383 us for gemm4's 266, fp4 K = 2240, N = 3877 at 1600
+// rows 46.1 for 36.5.
 struct MidCost { double once, per_round, per_fill, per_tile, split, row_mb; };
 constexpr MidCost kCost[4][3] = {   // by book; gemm4, 32 rows, 64 rows
     {{9.2, 1.386, 0.49, 5.4, 15.8, 0.0}, {10.0, 0.366, 0.0, 0.5, 1.6, 0.1173}, {14.5, 0.413, 0.151, 1.6, 2.4, 0.1145}},
