@@ -113,12 +113,12 @@ int rlq_linear_affine_kernel(int kernel, const void *x, int x_stride, int M, int
 /* The prefill GEMM is three kernels that give a row the same bits: FULL (128 x 256 output
  * tiles), MID32 and MID64 (32 or 64 rows x 128, calls with too few of those tiles) and FEW
  * (32 x 32, affine weights, a few rows). rlq_prefill_route returns the one a call of these
- * sizes runs (book 0 for affine weights; for a weight whose K is split, of its first rows;
- * 0 for sizes no call takes). The _prefill entry points run the one named, for tests and
+ * sizes runs (book 0 for affine weights, with the type of their scales, RLQ_F16 for native
+ * ones; for a weight whose K is split, of its first rows; 0 for sizes no call takes). The _prefill entry points run the one named, for tests and
  * measurement, with the contract of rlq_linear_affine; a kernel that cannot take the call
  * (FEW for native weights; too few counters for a split weight's tiles) is an error. */
 enum { RLQ_PREFILL_AUTO = 0, RLQ_PREFILL_FULL = 1, RLQ_PREFILL_MID32 = 2, RLQ_PREFILL_MID64 = 3, RLQ_PREFILL_FEW = 4 };
-int rlq_prefill_route(int book, int M, int K, int N);
+int rlq_prefill_route(int book, int scale_dtype, int M, int K, int N);
 int rlq_linear_affine_prefill(int route, const void *x, int x_stride, int M, int K, int N,
                               const void *packed, int scale_dtype,
                               float *y, int y_stride, int accum,

@@ -39,7 +39,7 @@ constexpr int kBiasProSteps = 11;
 enum PrefillRoute { kRouteAuto = 0, kRouteFull = 1, kRouteMid32 = 2, kRouteMid64 = 3, kRouteFew = 4 };
 
 // The route a call of these sizes takes (its first launch: a split weight's rows go in chunks).
-int prefill_route(int book, int M, int K, int N);
+int prefill_route(int book, int sd, int M, int K, int N);
 
 // route: kRouteAuto, or the kernel to run (an error where it cannot take the call).
 // codes, sbq: the two sections of a packed matrix (q4_tile.h), or of rows [r0, r0 + N) of a
@@ -52,13 +52,13 @@ int run_gemm4(int route, int book, const _Float16 *x, int x_stride, int M, int K
 // The kernel for calls with too few 128 x 256 tiles (gemm_mid.hip): gemm_mid_tiles gives the
 // 32-row tiles (1 or 2) of its workgroups' rows, or 0 where gemm4_kernel takes the call. Both
 // kernels give the same bits.
-int gemm_mid_tiles(int book, int M, int K, int N, int S);
+int gemm_mid_tiles(int book, int sd, int M, int K, int N, int S);
 bool gemm_mid_counters_fit(int mt, int M, int N, int S);   // a split launch's tiles have counters
 int launch_gemm_mid(int book, int sd, int mt, const GemmArgs &a, int S, int accum, hipStream_t st);
 
 // The affine kernel for a few rows (gemm_few.hip), the same bits again, and whether it takes a
 // call; a.x: the prepped activations by chunk, then row ([K / 8][M][8 halves]).
-bool gemm_few_fits(int M, int N, int S);
+bool gemm_few_fits(int M, int K, int N, int S);
 bool gemm_few_counters_fit(int M, int N, int S);
 int launch_gemm_few(int sd, const GemmArgs &a, int S, int accum, hipStream_t st);
 

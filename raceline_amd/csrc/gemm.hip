@@ -743,15 +743,15 @@ static int launch_gemm4_inst(int accum, dim3 grid, size_t lds, hipStream_t st, c
   return 0;
 }
 
-static int mid_route(int book, int M, int K, int N, int S) {
-  const int mt = gemm_mid_tiles(book, M, K, N, S);
+static int mid_route(int book, int sd, int M, int K, int N, int S) {
+  const int mt = gemm_mid_tiles(book, sd, M, K, N, S);
   return mt == 1 ? kRouteMid32 : mt == 2 ? kRouteMid64 : kRouteFull;
 }
 
-int prefill_route(int book, int M, int K, int N) {
+int prefill_route(int book, int sd, int M, int K, int N) {
   const int S = gemm_split_of(K, N);
-  if (book == kAffine && gemm_few_fits(M, N, S)) return kRouteFew;
-  return mid_route(book, S > 1 ? std::min(M, split_chunk_rows(N)) : M, K, N, S);
+  if (book == kAffine && gemm_few_fits(M, K, N, S)) return kRouteFew;
+  return mid_route(book, sd, S > 1 ? std::min(M, split_chunk_rows(N)) : M, K, N, S);
 }
 
 int run_gemm4(int route, int book, const _Float16 *x, int x_stride, int M, int K, int N, const void *codes,
@@ -779,7 +779,7 @@ int run_gemm4(int route, int book, const _Float16 *x, int x_stride, int M, int K
   RLQ_REQUIRE((route != kRouteMid32 && route != kRouteMid64) ||
                   gemm_mid_counters_fit(route == kRouteMid32 ? 1 : 2, std::min(M, chunk), N, S),
               "prefill kernel: route %d does not take M=%d N=%d split %d", route, M, N, S);
-  const bool few = route == kRouteAuto ? book == kAffine && gemm_few_fits(M, N, S) : route == kRouteFew;
+  const bool few = route == kRouteAuto ? book == kAffine && gemm_few_fits(M, K, N, S) : route == kRouteFew;
   if (book == kAffine) {
     const int gs_stride = gs_stride_of(G, sd);
     _Float16 *xp = static_cast<_Float16 *>(ws);
@@ -827,7 +827,7 @@ int run_gemm4(int route, int book, const _Float16 *x, int x_stride, int M, int K
       if (int rc = launch_gemm_few(sd, c, S, accum, st)) return rc;
       continue;
     }
-    const int r = route == kRouteAuto ? mid_route(book, c.M, K, N, S) : route;
+    const int r = route == kRouteAuto ? mid_route(book, sd, c.M, K, N, S) : route;
     if (r != kRouteFull) {   // too few of this kernel's tiles to fill the chip
       if (int rc = launch_gemm_mid(book, sd, r == kRouteMid32 ? 1 : 2, c, S, accum, st)) return rc;
       continue;

@@ -42,7 +42,7 @@ constexpr int kFewPairBytes = 2 * 4 * 1024;           // a pair's products: [gro
 constexpr int kFewScaleBytes = 512;                   // and its scale words: [lane] 8 bytes
 constexpr int kFewSetBytes = kFewProducers * (kFewPairBytes + kFewScaleBytes);
 constexpr int kFewMaxTiles = 256;                     // a workgroup per CU
-constexpr int kFewMaxRows = 2048;
+constexpr int kFewMaxRows = 2048, kFewShortK = 320;   // see gemm_few_fits
 constexpr int kFewLds = 2 * kFewSetBytes;             // 136 KB: one workgroup per CU
 
 // What a producer wave reads (see few_codes, few_frag).
@@ -315,10 +315,14 @@ __global__ __launch_bounds__(kFewThreads, 3) void gemm_few_kernel(GemmArgs a, in
 // pass writes each row's chunks 16 M bytes apart, eight rows to a cache line, which costs more
 // than the GEMM gains past about 2000 rows (f16 K = 2752 .. 13504, N = 21 .. 39: 3043 rows 35.1
 // us against 29.0, 3905 135.8 against 61.2, 8191 60.2 against 33.0; 1929 rows 27.1 against 28.0).
+// With a short K there is little to prepare (K = 192 .. 320: 3114 rows 12.8 against 14.2, 7915
+// 18.1 against 19.0; K = 512: 2843 rows 14.7 against 14.3).
 static long long few_tiles(int M, int N, int S, int rb) {
   return (long long)((N + 31) / 32) * ((M + rb - 1) / rb) * S;
 }
-bool gemm_few_fits(int M, int N, int S) { return M <= kFewMaxRows && few_tiles(M, N, S, 32) <= kFewMaxTiles; }
+bool gemm_few_fits(int M, int K, int N, int S) {
+  return (M <= kFewMaxRows || K <= kFewShortK) && few_tiles(M, N, S, 32) <= kFewMaxTiles;
+}
 bool gemm_few_counters_fit(int M, int N, int S) { return S == 1 || few_tiles(M, N, 1, 32) <= kGemmMaxCounters; }
 
 int launch_gemm_few(int sd, const GemmArgs &a, int S, int accum, hipStream_t st) {

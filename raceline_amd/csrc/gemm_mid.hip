@@ -422,10 +422,11 @@ static int launch_mid_rows(int mt, const GemmArgs &a, int S, int accum, hipStrea
 // Which kernel and tile take a call: the one of three estimated fastest (32 or 64 rows x 128
 // features here, gemm4_kernel's 128 x 256), each as, in us,
 //   once + pairs x (per_round x rounds of the chip + per_fill x fill) + (per_tile + split (S - 1)) x fill
-// with fill = units / units of a round, rounds = fill rounded up, and the group pairs of a
-// workgroup rounded up to the ones its loop runs (3, 8 or 4 LDS stages). A wave here is bound by
-// its own instruction issue, and two resident on a SIMD take about as long as one after the
-// other, so the rounds count; how full they are costs memory time and clock.
+// with fill = workgroups / CUs, rounds = fill rounded up, and the group pairs of a workgroup
+// rounded up to the ones its loop runs (3, 8 or 4 LDS stages). A wave here is bound by its own
+// instruction issue, and two workgroups on a CU take about as long as one after the other, so
+// the rounds count; how full they are costs memory time and clock. Past three rounds the CUs
+// drift apart, and a partial round counts half its empty part.
 // The tiles here have one more term. Each 128 features read all rows, which an XCD's L2 (4 MB)
 // holds for small calls; rows beyond it come from memory once per 128 features, at row_mb us per
 // MB (from 2 MB of rows on, in full from 12 MB). The native books' waves have little to do
@@ -433,48 +434,52 @@ static int launch_mid_rows(int mt, const GemmArgs &a, int S, int accum, hipStrea
 // the two (the cube root of the sum of cubes). gemm4_kernel orders its tiles in blocks of 512
 // rows and shows no such term.
 // The books differ in what a code costs to convert (4 operations for eight fp4 codes, 13 for
-// eight integer ones, shared by two row tiles at 64 rows), the affine one in its scale FMAs,
-// int16 in the launch that sums its rows first. Fitted to launches timed with their prep pass:
-// K 128 .. 17408 (odd numbers of groups and split weights among them), N 16 .. 34816, 9 .. 4096
-// rows (to 16384 where N < 256), 828 calls (affine), 431 (int15), 467 (int16) and 470 (fp4).
-// Against the fastest of the three the choice loses 0.3%, 0.1%, 0.3% and 0.4% on average and at
-// most 11%, 16%, 20% and 19%. Of these calls and 1423 others drawn afterwards three are slower
-// than on gemm4_kernel alone as it was before the tiles here (1.4%, 1.5% and 3.1%). Without the
-// rows' term, the rounding of the pairs and the split it took the 64-row tiles for large calls:
-// bf16 K = 16512, N = 2187 at 2762 rows 383 us for gemm4's 266, fp4 K = 2240, N = 3877 at 1600
-// rows 46.1 for 36.5.
+// eight integer ones, shared by two row tiles at 64 rows), the affine ones in their scale FMAs
+// and bias steps (twice as many for bf16), int16 in the launch that sums its rows first. Fitted
+// to launches timed with their prep pass: K 128 .. 17408 (odd numbers of groups and split
+// weights among them), N 16 .. 34816, 9 .. 4096 rows (to 16384 where N < 256), 600 to 734 calls
+// a book. Against the fastest of the three the choice loses 0.2% (affine), 0.1% (integer books)
+// and 0.3% (fp4) on average, and 4%, 5% and 6% at 99 of 100 calls. Without the rows' term, the
+// rounding of the pairs and the split it took the 64-row tiles for large calls and was slower
+// than gemm4_kernel alone: bf16 K = 16512, N = 2187 at 2762 rows 383 us for 266, fp4 K = 2240,
+// N = 3877 at 1600 rows 46.1 for 36.5.
 struct MidCost { double once, per_round, per_fill, per_tile, split, row_mb; };
-constexpr MidCost kCost[4][3] = {   // by book; gemm4, 32 rows, 64 rows
-    {{9.2, 1.386, 0.49, 5.4, 15.8, 0.0}, {10.0, 0.366, 0.0, 0.5, 1.6, 0.1173}, {14.5, 0.413, 0.151, 1.6, 2.4, 0.1145}},
-    {{4.0, 1.214, 0.339, 7.6, 9.5, 0.0}, {5.0, 0.349, 0.0, 0.4, 0.6, 0.0057}, {4.5, 0.478, 0.0, 1.6, 2.0, 0.0118}},
-    {{10.5, 1.253, 0.557, 4.5, 15.7, 0.0}, {8.3, 0.356, 0.0, 0.3, 2.9, 0.013}, {7.9, 0.489, 0.0, 1.4, 3.7, 0.0158}},
-    {{4.6, 1.03, 0.421, 7.5, 8.2, 0.0}, {4.1, 0.212, 0.016, 1.1, 0.0, 0.0238}, {4.2, 0.336, 0.016, 2.4, 0.2, 0.0248}}};
+constexpr MidCost kCost[5][3] = {   // affine with fp16 scales, int15, int16, fp4, affine with bf16 scales: gemm4, 32 rows, 64 rows
+    {{10.4, 1.353, 0.537, 1.9, 20.2, 0}, {9.3, 0.359, 0.022, 1.1, 2.2, 0.0997}, {12.5, 0.511, 0.003, 3, 3.8, 0.1117}},
+    {{4.4, 1.161, 0.477, 5.9, 8.6, 0}, {4.7, 0.358, 0.009, 0.4, 0.6, 0.001}, {4.3, 0.47, 0.004, 1.7, 0, 0.0193}},
+    {{9.6, 1.207, 0.55, 5, 15.2, 0}, {7.9, 0.368, 0, 0.4, 2.7, 0.0073}, {7.6, 0.476, 0.008, 1.5, 3.4, 0.0171}},
+    {{4, 1.016, 0.521, 5.9, 5.8, 0}, {4.3, 0.216, 0.023, 1.1, 1.5, 0.0229}, {4, 0.335, 0.046, 2, 0.2, 0.0206}},
+    {{8.4, 1.447, 0.482, 5.6, 11.1, 0}, {8.5, 0.372, 0.029, 1.4, 0.9, 0.1222}, {12.3, 0.561, 0.003, 2.6, 0.7, 0.0953}}};
 static_assert(kAffine == 0 && kInt15 == 1 && kInt16 == 2 && kFp4 == 3, "kCost's rows");
-// what gemm4_kernel may be slower by and still take a call: estimates closer than this pick
-// either, and its times vary less
-constexpr double kMidMargin = 1.02;
+// Ties: what gemm4_kernel may be estimated slower by and still take a call, the margin that left
+// the fewest calls slower than on the kernel they ran before (between boxes the two differ by
+// 5% either way, as the clock does).
+constexpr double mid_margin(int book) { return book == kInt15 || book == kInt16 ? 0.99 : 1.02; }
 
 // a split call's tiles count their arrivals in the workspace's counters
 bool gemm_mid_counters_fit(int mt, int M, int N, int S) {
   return S == 1 || (long long)((M + 32 * mt - 1) / (32 * mt)) * ((N + kMidCols - 1) / kMidCols) <= kGemmMaxCounters;
 }
 
-int gemm_mid_tiles(int book, int M, int K, int N, int S) {
+int gemm_mid_tiles(int book, int sd, int M, int K, int N, int S) {
   const int pairs = ((K / kGroup + 1) / 2 + S - 1) / S;
   const double rows_mb = 2e-6 * M * K, beyond = std::clamp((rows_mb - 2.0) / 10.0, 0.0, 1.0);
   const double read = rows_mb * ((N + kMidCols - 1) / kMidCols) * beyond;
-  auto time = [&](const MidCost &c, long long units, int per, int stages) {
-    const double fill = (double)units / per, rounds = (double)((units + per - 1) / per);
+  const MidCost *cost = kCost[book == kAffine && sd == RLQ_BF16 ? 4 : book];
+  // the kernel of cost[i]: workgroups of rows x cols, and the pairs of one turn of its loop
+  auto time = [&](int i, int rows, int cols, int stages) {
+    const MidCost &c = cost[i];
+    const long long wgs = (long long)((N + cols - 1) / cols) * ((M + rows - 1) / rows) * S;
+    const double fill = wgs / 256.0, whole = (double)((wgs + 255) / 256);
+    const double rounds = i > 0 && fill > 3.0 ? 0.5 * (whole + fill) : whole;
     const double run = (double)((pairs + stages - 1) / stages * stages);
     const double work = run * (c.per_round * rounds + c.per_fill * fill) + (c.per_tile + c.split * (S - 1)) * fill;
-    const double rows = c.row_mb * read;
-    return c.once + (book == kAffine ? std::cbrt(work * work * work + rows * rows * rows) : work + rows);
+    const double mem = c.row_mb * read;
+    return c.once + (book == kAffine ? std::cbrt(work * work * work + mem * mem * mem) : work + mem);
   };
-  const MidCost *cost = kCost[book];
-  const long long nt = (N + 31) / 32;
-  const double t4 = time(cost[0], (long long)((N + 255) / 256) * ((M + 127) / 128) * S, 256, 3);
-  const double t1 = kMidMargin * time(cost[1], nt * ((M + 31) / 32) * S, 1024, mid_ring<1>());
-  const double t2 = kMidMargin * time(cost[2], nt * ((M + 63) / 64) * S, 1024, mid_ring<2>());
+  const double t4 = time(0, 128, 256, 3);
+  const double t1 = mid_margin(book) * time(1, 32, kMidCols, mid_ring<1>());
+  const double t2 = mid_margin(book) * time(2, 64, kMidCols, mid_ring<2>());
   if (t1 <= t2 && t1 < t4 && gemm_mid_counters_fit(1, M, N, S)) return 1;
   return t2 < t4 && gemm_mid_counters_fit(2, M, N, S) ? 2 : 0;
 }

@@ -1001,9 +1001,11 @@ size_t rlq_linear_workspace_bytes(int M, int K, int N) {
                                      gemm4_workspace(kInt16, M, K, N), gemm4_workspace(kInt15, M, K, N)});
 }
 
-int rlq_prefill_route(int book, int M, int K, int N) {
-  if (M <= 0 || N <= 0 || K <= 0 || K % kGroup || book < kAffine || book > kFp4) return 0;
-  return prefill_route(book, M, K, N);
+int rlq_prefill_route(int book, int scale_dtype, int M, int K, int N) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % kGroup || book < kAffine || book > kFp4 ||
+      (scale_dtype != RLQ_F16 && scale_dtype != RLQ_BF16))
+    return 0;
+  return prefill_route(book, scale_dtype, M, K, N);
 }
 
 static int linear_affine(int kernel, const void *x, int x_stride, int M, int K, int N, const void *packed,

@@ -35,7 +35,7 @@ SIGNATURES = {
                                   c_void_p, c_size_t, c_void_p]),
     "rlq_linear_affine_kernel": (c_int, [c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p,
                                          c_int, c_int, c_void_p, c_size_t, c_void_p]),
-    "rlq_prefill_route": (c_int, [c_int, c_int, c_int, c_int]),
+    "rlq_prefill_route": (c_int, [c_int, c_int, c_int, c_int, c_int]),
     "rlq_linear_affine_prefill": (c_int, [c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p,
                                           c_int, c_int, c_void_p, c_size_t, c_void_p]),
     "rlq_linear_native_prefill": (c_int, [c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int,

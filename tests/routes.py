@@ -7,11 +7,11 @@ AFFINE = (FULL, MID32, MID64, FEW)
 NATIVE = (FULL, MID32, MID64)
 
 
-def chosen(book, M, K, N):
+def chosen(book, M, K, N, scale_dtype=0):
     """The kernel a call of these sizes runs; book: 0 (affine) or the native codebook's code."""
     from raceline_amd import lib
 
-    return lib.call("rlq_prefill_route", book, M, K, N)
+    return lib.call("rlq_prefill_route", book, scale_dtype, M, K, N)
 
 
 def linear_on(route, x, w, out=None, accum=False):

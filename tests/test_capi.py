@@ -140,38 +140,45 @@ def test_prefill_kernel_that_cannot_take_the_call_is_refused():
             lib.call("rlq_linear_affine_prefill", route, *split)
         with pytest.raises(lib.RlqError, match="unknown route"):
             lib.call("rlq_linear_native_prefill", route, *native)
-    assert lib.call("rlq_prefill_route", 0, 64, 100, 64) == 0
-    assert lib.call("rlq_prefill_route", 4, 64, 128, 64) == 0
+    assert lib.call("rlq_prefill_route", 0, 0, 64, 100, 64) == 0
+    assert lib.call("rlq_prefill_route", 4, 0, 64, 128, 64) == 0
+    assert lib.call("rlq_prefill_route", 0, 2, 64, 128, 64) == 0
 
 
 def test_prefill_kernel_of_tall_narrow_calls():
-    """The few-row kernel takes calls of at most 256 tiles of 32 x 32 and 2048 rows: with more
-    rows its prep pass costs more than it gains (3905 x 13504 x 21: 136 us against 61)."""
+    """The few-row kernel takes calls of at most 256 tiles of 32 x 32 and, unless K is short,
+    2048 rows: with more rows its prep pass costs more than it gains (3905 x 13504 x 21: 136 us
+    against 61)."""
     def route(M, K, N):
-        return lib.call("rlq_prefill_route", 0, M, K, N)
+        return lib.call("rlq_prefill_route", 0, 0, M, K, N)
 
-    assert all(route(*c) == 4 for c in ((9, 4096, 4096), (64, 4096, 4096), (2048, 4096, 64), (1024, 512, 256)))
+    assert all(route(*c) == 4 for c in ((9, 4096, 4096), (64, 4096, 4096), (2048, 4096, 64), (1024, 512, 256),
+                                        (8192, 320, 32)))
     assert all(route(*c) in (1, 2, 3) for c in ((65, 4096, 4096), (2049, 4096, 32), (3905, 13504, 21), (8192, 4096, 32)))
 
 
-# book, M, K, N and the prefill kernels that are the fastest there or within a few percent of it
-# (1 full tiles, 2 and 3 tiles of 32 and 64 rows), all timed on the same weights: large calls,
-# whose rows outgrow an L2, as the full tiles' (3 to 44% slower on 64-row tiles), small and
-# mid-size ones on the others (full tiles 1.2 to 3 times slower), short K and split weights
+# book, scale type, M, K, N and the prefill kernels that are the fastest there or within a few
+# percent of it (1 full tiles, 2 and 3 tiles of 32 and 64 rows), all timed on the same weights:
+# large calls, whose rows outgrow an L2, as the full tiles' (3 to 44% slower on 64-row tiles),
+# small and mid-size ones on the others (full tiles 1.1 to 3 times slower), short K, split
+# weights, and a partial last round after many
 PREFILL_CHOICES = [
-    (0, 2762, 16512, 2187, (1,)), (0, 1329, 10240, 3841, (1,)), (0, 1600, 5120, 7168, (1,)), (0, 841, 8000, 5104, (1,)),
-    (0, 1887, 8192, 2466, (1,)), (0, 2048, 5120, 34816, (1,)), (1, 2048, 4096, 6144, (1,)), (1, 2393, 9408, 2330, (1,)),
-    (1, 3591, 2624, 3106, (1,)), (3, 2048, 4096, 6144, (1,)), (3, 1600, 2240, 3877, (1,)),
-    (3, 1904, 15744, 2529, (1,)), (3, 2037, 5824, 2750, (1,)),
-    (0, 100, 4096, 4096, (2,)), (0, 300, 5120, 7168, (2,)), (0, 1024, 4096, 4096, (2, 3)), (0, 200, 17408, 5120, (2, 3)),
-    (0, 2048, 5120, 5120, (3,)), (1, 20, 320, 254, (2, 3)), (1, 512, 5120, 34816, (1, 3)), (2, 104, 192, 1540, (2, 3)),
-    (2, 17, 192, 20, (2, 3)), (3, 64, 4096, 24576, (2, 3)), (3, 700, 4096, 4096, (2, 3)), (3, 1024, 4096, 4096, (2, 3))]
+    (0, 1, 2762, 16512, 2187, (1,)), (0, 1, 1329, 10240, 3841, (1,)), (0, 1, 1600, 5120, 7168, (1,)),
+    (0, 1, 841, 8000, 5104, (1,)), (0, 0, 1887, 8192, 2466, (1,)), (0, 0, 2048, 5120, 34816, (1,)),
+    (0, 1, 327, 1024, 11428, (1,)), (1, 0, 2048, 4096, 6144, (1,)), (1, 0, 2393, 9408, 2330, (1,)),
+    (1, 0, 3591, 2624, 3106, (1,)), (3, 0, 2048, 4096, 6144, (1,)), (3, 0, 1600, 2240, 3877, (1,)),
+    (3, 0, 1904, 15744, 2529, (1,)), (3, 0, 2037, 5824, 2750, (1,)),
+    (0, 0, 100, 4096, 4096, (2,)), (0, 1, 300, 5120, 7168, (2,)), (0, 0, 1024, 4096, 4096, (2, 3)),
+    (0, 1, 200, 17408, 5120, (2, 3)), (0, 0, 2048, 5120, 5120, (3,)),
+    (1, 0, 20, 320, 254, (2, 3)), (1, 0, 1024, 4096, 6144, (1, 3)), (1, 0, 1112, 2688, 7454, (3,)),
+    (2, 0, 104, 192, 1540, (2, 3)), (2, 0, 17, 192, 20, (2, 3)), (3, 0, 64, 4096, 24576, (2, 3)),
+    (3, 0, 700, 4096, 4096, (2, 3)), (3, 0, 1024, 4096, 4096, (2, 3))]
 
 
 def test_prefill_kernel_choice():
     """The kernel a prefill call takes is one of those measured fastest, over sizes and books."""
-    wrong = [c for c in PREFILL_CHOICES if lib.call("rlq_prefill_route", *c[:4]) not in c[4]]
-    assert not wrong, [(c, lib.call("rlq_prefill_route", *c[:4])) for c in wrong]
+    wrong = [(c, r) for c in PREFILL_CHOICES if (r := lib.call("rlq_prefill_route", *c[:5])) not in c[5]]
+    assert not wrong, wrong
 
 
 def test_calls_follow_a_reloaded_library(tmp_path, monkeypatch):
